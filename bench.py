@@ -36,10 +36,10 @@ sys.path.insert(0, ROOT)
 
 METRIC = "RGF energy-points/s @nb=512×100 slabs: FP64 vs mixed+warm-start @≤1e-8 err"
 # complex products and inversions run per slab of a ballistic sweep, 8 n^3 flops
-# each: pass 1 five products and the inversion, pass 2 seven products between
-# slabs of equal size (eight otherwise)
-SLAB_FLOPS_EQUAL = 13 * 8
-SLAB_FLOPS_UNEVEN = 14 * 8
+# each: pass 1 five products and the inversion, pass 2 five products between
+# slabs of equal size (seven otherwise)
+SLAB_FLOPS_EQUAL = 11 * 8
+SLAB_FLOPS_UNEVEN = 13 * 8
 PEAK_FP64 = 78.6  # TFLOP/s, MI355X dense FP64 matrix
 # HBM bytes moved by one 512^3 complex product without an addend (A and B read
 # once, C written once), measured with rocprofv3 FETCH_SIZE / WRITE_SIZE and a

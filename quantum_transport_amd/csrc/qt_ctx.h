@@ -25,6 +25,7 @@ struct qt_ham {
     double2* S = nullptr;       // [nk][hset] or null (identity)
     bool uniform = true;
     bool leads_same = false;    // both contacts are the same semi-infinite lead
+    std::vector<char> csame;    // coupling s equals coupling s - 1 in every k set (s >= 1)
     int nmax = 0;
 };
 
@@ -148,6 +149,8 @@ struct Work {
     double2* Gln = nullptr;
     double2* H00 = nullptr;  // Hii + sigma_r S per point (only with sigma), same layout
     double2* SLS = nullptr;  // sigma_lesser S per point (only with sigma), same layout
+    double2* X = nullptr;    // Gl U^H of every pass-1 step through coupling c, at coff[c]*B (or null)
+    double2* V = nullptr;    // Gl U of the same steps (without sigma; or null)
     double2* T[NTEMP];       // temps, 2B * nn each
     double2* sigF = nullptr; // first-contact self-energy [B][nn]
     double2* sigL = nullptr; // last-contact self-energy  [B][nn]
@@ -175,8 +178,9 @@ struct Work {
     double2* diag = nullptr;    // 3 * B * ndiag staging
 };
 
-size_t work_bytes(const qt_ham& h, int B, bool sigma);
-void work_carve(Arena& a, Work& w, const qt_ham& h, int B, bool sigma);
+// keep: the first pass's coupling products stay resident for the second one
+size_t work_bytes(const qt_ham& h, int B, bool sigma, bool keep = false);
+void work_carve(Arena& a, Work& w, const qt_ham& h, int B, bool sigma, bool keep = false);
 void inv_batch(Ctx& c, Work& w, int n, int batch, double2* A, int64_t sa, double2* X, int64_t sx,
                const int* active, int flop_batch = -1);
 void note_inv_info(Ctx& c, Work& w, int batch, int period);

@@ -191,6 +191,54 @@ __global__ void diag_kernel(DiagArgs a) {
     if (a.gg) a.gg[o] = make_double2(l.x, l.y + 2.0 * g.y);  // G - G^H on the diagonal = 2i Im G
 }
 
+// Diagonals of G = Gc + Z Gc without the product: G[j,j] = Gc[j,j] +
+// sum_k Z[j,k] Gc[k,j].  A workgroup takes 32 columns j and walks k in tiles of
+// 32, both read along their columns; Z's tile is turned in LDS.  Bound by the
+// one read of Z and Gc: 32 n^2 bytes a member where the product costs
+// 8 n^3 flops.
+__global__ __launch_bounds__(256) void diag_z_kernel(DiagArgs a, ZOp Zo) {
+    const int b = blockIdx.y, n = a.n;
+    if (a.active && !a.active[b]) return;
+    const double2* __restrict__ G = a.G.p + b * a.G.sb;
+    const double2* __restrict__ Z = Zo.p + b * Zo.sb;
+    __shared__ double2 tz[TT][TT + 1], tg[TT][TT + 1];
+    __shared__ double2 part[8][TT];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5, j0 = blockIdx.x * TT;
+    double re = 0.0, im = 0.0;  // column j0 + tx, the k of this tile row group
+    for (int k0 = 0; k0 < n; k0 += TT) {
+        for (int r = ty; r < TT; r += 8) {
+            const bool okz = j0 + tx < n && k0 + r < n, okg = k0 + tx < n && j0 + r < n;
+            tz[r][tx] = okz ? Z[j0 + tx + (int64_t)(k0 + r) * Zo.ld] : make_double2(0.0, 0.0);
+            tg[r][tx] = okg ? G[k0 + tx + (int64_t)(j0 + r) * a.G.ld] : make_double2(0.0, 0.0);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < TT / 8; ++q) {
+            const int k = ty + 8 * q;
+            const double2 z = tz[k][tx], g = tg[tx][k];  // Z[j, k0 + k], Gc[k0 + k, j]
+            re = fma(z.x, g.x, re);
+            re = fma(-z.y, g.y, re);
+            im = fma(z.x, g.y, im);
+            im = fma(z.y, g.x, im);
+        }
+        __syncthreads();
+    }
+    part[ty][tx] = make_double2(re, im);
+    __syncthreads();
+    const int j = j0 + tx;
+    if (ty != 0 || j >= n) return;
+    double2 g = G[j + (int64_t)j * a.G.ld];
+    for (int q = 0; q < 8; ++q) {
+        g.x += part[q][tx].x;
+        g.y += part[q][tx].y;
+    }
+    const double2 l = a.Gl.p[b * a.Gl.sb + j + (int64_t)j * a.Gl.ld];
+    const int64_t o = b * a.ld + a.off + j;
+    if (a.gr) a.gr[o] = g;
+    if (a.gl) a.gl[o] = l;
+    if (a.gg) a.gg[o] = make_double2(l.x, l.y + 2.0 * g.y);  // G - G^H on the diagonal = 2i Im G
+}
+
 // ---------------------------------------------------------------- Sancho step
 __device__ __forceinline__ double block_sum(double v, double* red) {
     red[threadIdx.x] = v;
@@ -379,6 +427,12 @@ void contact_current(hipStream_t s, const CurrentArgs& a) {
 void diag_extract(hipStream_t s, const DiagArgs& a) {
     if (a.batch <= 0) return;
     hipLaunchKernelGGL(diag_kernel, dim3((a.n + 255) / 256, a.batch), dim3(256), 0, s, a);
+    QT_HIP(hipGetLastError());
+}
+
+void diag_extract_z(hipStream_t s, const DiagArgs& a, ZOp Z) {
+    if (a.batch <= 0) return;
+    hipLaunchKernelGGL(diag_z_kernel, dim3((a.n + TT - 1) / TT, a.batch), dim3(256), 0, s, a, Z);
     QT_HIP(hipGetLastError());
 }
 

@@ -147,6 +147,8 @@ struct DiagArgs {
     const int* active = nullptr;
 };
 void diag_extract(hipStream_t s, const DiagArgs& a);
+// the same with G = Gc + Z Gc given by its factors: G takes Gc, Z n x n blocks
+void diag_extract_z(hipStream_t s, const DiagArgs& a, ZOp Z);
 
 // Sancho-Rubio step update (rgf_mod.f90:526-541):
 //   H_SS += C; H_BB += C + Ap; err_b = sum |H01n|; converged when err < tol

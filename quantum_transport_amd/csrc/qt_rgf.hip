@@ -51,12 +51,13 @@ static int prec_digits(int precision) {
     }
 }
 
-size_t work_bytes(const qt_ham& h, int B, bool sigma) {
+size_t work_bytes(const qt_ham& h, int B, bool sigma, bool keep) {
     const int64_t nn = (int64_t)h.nmax * h.nmax;
     const int64_t tiles = (h.nmax + 31) / 32;
     size_t b = 0;
     auto add = [&](size_t bytes) { b += (bytes + 255) & ~size_t(255); };
     add(sizeof(double2) * (size_t)h.hset * B * (sigma ? 4 : 2));
+    if (keep) add(sizeof(double2) * (size_t)h.cset * B * (sigma ? 1 : 2) + 256);
     for (int i = 0; i < NTEMP; ++i) add(sizeof(double2) * (size_t)nn * 2 * B);
     add(sizeof(double2) * (size_t)nn * B * 2);
     add(sizeof(int) * (size_t)2 * B * h.nmax);
@@ -69,7 +70,7 @@ size_t work_bytes(const qt_ham& h, int B, bool sigma) {
     return b + (1 << 20);
 }
 
-void work_carve(Arena& a, Work& w, const qt_ham& h, int B, bool sigma) {
+void work_carve(Arena& a, Work& w, const qt_ham& h, int B, bool sigma, bool keep) {
     a.reset();
     w.B = B;
     w.nmax = h.nmax;
@@ -81,6 +82,8 @@ void work_carve(Arena& a, Work& w, const qt_ham& h, int B, bool sigma) {
     w.Gln = a.take<double2>((size_t)h.hset * B);
     w.H00 = sigma ? a.take<double2>((size_t)h.hset * B) : nullptr;
     w.SLS = sigma ? a.take<double2>((size_t)h.hset * B) : nullptr;
+    w.X = keep ? a.take<double2>((size_t)h.cset * B) : nullptr;
+    w.V = keep && !sigma ? a.take<double2>((size_t)h.cset * B) : nullptr;
     for (int i = 0; i < NTEMP; ++i) w.T[i] = a.take<double2>((size_t)w.nn * 2 * B);
     w.sigF = a.take<double2>((size_t)w.nn * B);
     w.sigL = a.take<double2>((size_t)w.nn * B);
@@ -385,18 +388,42 @@ struct Solve {
         return op_member(w.SLS + h.hoff[s] * B, h.nm[s], sq(s));
     }
 
-    void diag_out(int s, const double2* G, const double2* L) {
+    // X = Gl U^H of the pass-1 step through coupling c: kept, or a temporary
+    double2* xbuf(int c) const { return w.X ? w.X + h.coff[c] * B : w.T[0]; }
+    int64_t xstr(int c) const { return w.X ? (int64_t)h.nm[c] * h.nm[c - 1] : w.nn; }
+    // the second pass couples slab sc to its solved neighbour through the block
+    // the first pass went through (backward, or with QT_F_COUPLING_FIX), or
+    // through the next lower one (the reference's forward variant)
+    int step_coupling(int sc) const { return fwd ? sc + 1 : sc; }
+    bool kept(int sc) const {
+        const int cc = step_coupling(sc);
+        return w.X && (!fwd || fix || h.csame[cc]);
+    }
+    // Z form between slabs of equal size: the blocks X G W Gl and X G W Gln come
+    // from Z = X (G W).  Between unequal ones the products W Gl and W Gln stay
+    // (with Z the contact current lost up to a factor three of its accuracy
+    // next to band edges, and 1% of the time was all it gave).  The choice
+    // depends on the sizes only, so a point's results do not depend on the
+    // outputs requested.
+    bool zform(int sc) const { return h.nm[sc] == h.nm[fwd ? sc + 1 : sc - 1]; }
+
+    // diagonals of slab s from G and G^<, or (Z given) from Gl, Z and G^<
+    void diag_out(int s, const double2* G, const double2* L, const double2* Z = nullptr) {
+        if (!gr && !glo && !gg) return;
         DiagArgs d;
         d.n = h.nm[s];
         d.batch = B;
-        d.G = op_member(G, h.nm[s], w.nn);
+        d.G = Z ? opGl(s) : op_member(G, h.nm[s], w.nn);
         d.Gl = op_member(L, h.nm[s], w.nn);
         d.gr = gr;
         d.gl = glo;
         d.gg = gg;
         d.ld = w.ndiag;
         d.off = doff[s];
-        diag_extract(c.stream, d);
+        if (Z)
+            diag_extract_z(c.stream, d, op_member(Z, h.nm[s], w.nn));
+        else
+            diag_extract(c.stream, d);
     }
 
     // G_r, G_lesser, G_greater (and Jdens from `jd`) of slab s to the host
@@ -436,7 +463,7 @@ struct Solve {
     //   GLi1 = G<_{l,l+1} = Y - (Gc Q)^H          (Gln anti-Hermitian)
     //   A    = G<_{l+1,l} = Lc X^H + Gc Q
     //   cur  = Re(W^H A) - Re(W GLi1),  GRi1 = GN0,  GGi1 = Gl^H W^H G^>_last
-    void gw_extras(int sc, int n, const ZOp& W, double2* X, double2* Y, double2* Q, double2* GN0,
+    void gw_extras(int sc, int n, const ZOp& W, const ZOp& X, double2* Y, double2* Q, double2* GN0,
                    double2* Gc, double2* Lc, const Gemm& g) {
         hipStream_t s = c.stream;
         const int64_t nn = w.nn;
@@ -459,7 +486,7 @@ struct Solve {
         an.Z = op_member(R, n, nn);
         an.c2 = -1.0;
         antiherm(s, an);
-        g(OP_N, OP_C, n, n, n, op_member(Lc, n, nn), op_member(X, n, nn), Acur, n, nn, 1.0,
+        g(OP_N, OP_C, n, n, n, op_member(Lc, n, nn), X, Acur, n, nn, 1.0,
           op_member(R, n, nn), 1.0);                                                    // Lc X^H + Gc Q
         if (full.cur) {
             g(OP_C, OP_N, n, n, n, W, op_member(Acur, n, nn), P1, n, nn);
@@ -607,8 +634,9 @@ struct Solve {
         int sp = sf;
         for (int sc = sf + step; sc != sl; sc += step) {
             const int n = h.nm[sc], np = h.nm[sp];
-            const ZOp U = opC(fwd ? sc : sc + 1);  // H1i(ii) forward, H1i(ii+1) backward
-            g(OP_N, OP_N, n, np, np, U, opGl(sp), T[0], n, nn);          // U Gl
+            const int cc = fwd ? sc : sc + 1;
+            const ZOp U = opC(cc);  // H1i(ii) forward, H1i(ii+1) backward
+            g(OP_N, OP_C, np, n, np, opGl(sp), U, xbuf(cc), np, xstr(cc));  // X = Gl U^H
             ShiftArgs sh;
             sh.n = n;
             sh.batch = B;
@@ -620,7 +648,7 @@ struct Solve {
             sh.c1 = -1.0;
             sh.kidx = w.kidx;
             shifted(s, sh);                                              // z S - H00
-            g(OP_N, OP_C, n, n, np, op_member(T[0], n, nn), U, T[1], n, nn, -1.0,
+            g(OP_N, OP_N, n, n, np, U, op_member(xbuf(cc), np, xstr(cc)), T[1], n, nn, -1.0,
               op_member(T[1], n, nn), 1.0);                              // - U Gl U^H
             inv_batch(c, w, n, B, T[1], nn, gl(sc), sq(sc), nullptr);
             note_inv_info(c, w, B, B);
@@ -633,9 +661,11 @@ struct Solve {
             } else {
                 // no interior injection: Gln = Gl U Gln' U^H Gl^H = V Gln' V^H with
                 // V = Gl U, three products instead of four
-                g(OP_N, OP_N, n, np, n, opGl(sc), U, T[2], n, nn);       // V = Gl U
-                g(OP_N, OP_N, n, np, np, op_member(T[2], n, nn), opGln(sp), T[3], n, nn);
-                g(OP_N, OP_C, n, n, np, op_member(T[3], n, nn), op_member(T[2], n, nn), gln(sc), n,
+                double2* V = w.V ? w.V + h.coff[cc] * B : T[2];
+                const int64_t sv = w.V ? (int64_t)n * np : nn;
+                g(OP_N, OP_N, n, np, n, opGl(sc), U, V, n, sv);          // V = Gl U
+                g(OP_N, OP_N, n, np, np, op_member(V, n, sv), opGln(sp), T[3], n, nn);
+                g(OP_N, OP_C, n, n, np, op_member(T[3], n, nn), op_member(V, n, sv), gln(sc), n,
                   sq(sc));                                               // (V Gln') V^H
             }
             sp = sc;
@@ -647,8 +677,9 @@ struct Solve {
         double2* Ln = T[9];
         {
             const int n = nL, np = h.nm[sp];
-            const ZOp U = opC(fwd ? sl : sl + 1);
-            g(OP_N, OP_N, n, np, np, U, opGl(sp), T[0], n, nn);
+            const int cc = fwd ? sl : sl + 1;
+            const ZOp U = opC(cc);
+            g(OP_N, OP_C, np, n, np, opGl(sp), U, xbuf(cc), np, xstr(cc));  // X = Gl U^H
             ShiftArgs sh;
             sh.n = n;
             sh.batch = B;
@@ -662,7 +693,7 @@ struct Solve {
             sh.c2 = -1.0;
             sh.kidx = w.kidx;
             shifted(s, sh);                                              // z S - H00 - Sigma
-            g(OP_N, OP_C, n, n, np, op_member(T[0], n, nn), U, T[1], n, nn, -1.0,
+            g(OP_N, OP_N, n, n, np, U, op_member(xbuf(cc), np, xstr(cc)), T[1], n, nn, -1.0,
               op_member(T[1], n, nn), 1.0);                              // - U Gl U^H
             inv_batch(c, w, n, B, T[1], nn, Gc, nn, nullptr);
             note_inv_info(c, w, B, B);
@@ -735,40 +766,59 @@ struct Solve {
         QT_HIP(hipEventRecord(c.ev[2], s));
 
         // ---------------- pass 2 (rgf_mod.f90:212-250 / 420-458)
+        // With Z_i = X_i G_{i+1} W the full block is G_i = (I + Z_i) Gl_i, and G
+        // itself is not needed to go on: G_i W = V_i + Z_i V_i with the V_i = Gl_i U
+        // of the first pass.  So where only diagonals are asked for, a slab takes
+        // five products here (ten in all, with the inversion) instead of seven, G
+        // being formed at the contact, for callers that want its blocks, and
+        // where the next slab needs it.  Measured, whole
+        // sweeps (leads included): 512 x 20 slabs, 64 points 482.7 -> 446.3 ms; the GW
+        // recursion with its Sigma, 96 x 4 slabs, 256 energies, 44.9 -> 38.1 ms an
+        // iteration.
         int sn = sl;
+        double2 *Zc = T[6] + B * nn, *Zn = T[7] + B * nn;  // Z of the solved neighbour and of this slab
+        bool haveZ = false;
         for (int sc = sl - step; sc != sf - step; sc -= step) {
             const int n = h.nm[sc], nq = h.nm[sn];
             // coupling between slab sc and its solved neighbour: the reference
             // uses H1i(ii) in both variants; QT_F_COUPLING_FIX selects H1i(ii+1)
             // in the forward variant
             const ZOp W = opC(fwd && fix ? sc + 1 : sc);  // nq x n
-            double2 *X = T[0], *GN0 = T[1], *P = T[2], *Y = T[3], *Q = T[4], *U = T[5];
-            // Z form: GN0 (W Gl) and GN0 (W Gln) as (GN0 W) Gl and (GN0 W) Gln,
-            // three products instead of four, between slabs of equal size (the
-            // RGF variants; the GW variant keeps GN0 and Q for its extra
-            // blocks).  The choice depends on the device and the variant only,
-            // so a point's results do not depend on the outputs requested.
-            const bool zform = !gw && nq == n;
-            double2* Z = P;  // n x n, ld n
-            g(OP_N, OP_C, n, nq, n, opGl(sc), W, X, n, nn);                                   // X = Gl W^H
-            g(OP_N, OP_N, n, nq, nq, op_member(X, n, nn), op_member(Gc, nq, nn), GN0, n, nn);  // GN0 = X G
-            if (zform) {
-                g(OP_N, OP_N, n, n, nq, op_member(GN0, n, nn), W, Z, n, nn);                  // Z = GN0 W
-                g(OP_N, OP_N, n, n, n, op_member(Z, n, nn), opGl(sc), Gn, n, nn, 1.0, opGl(sc),
-                  1.0);                                                                        // G = Gl + Z Gl
+            const int cc = step_coupling(sc);
+            const bool kx = kept(sc), zf = zform(sc);
+            double2 *GN0 = T[1], *P = T[2], *Y = T[3], *Q = T[4], *U = T[5];
+            double2* Xb = kx ? xbuf(cc) : T[0];
+            const ZOp X = op_member(Xb, n, kx ? xstr(cc) : nn);
+            if (!kx) g(OP_N, OP_C, n, nq, n, opGl(sc), W, Xb, n, nn);                          // X = Gl W^H
+            if (!zf || want_gw)
+                g(OP_N, OP_N, n, nq, nq, X, op_member(Gc, nq, nn), GN0, n, nn);               // GN0 = X G
+            if (zf) {
+                if (haveZ && kx && w.V) {
+                    const ZOp V = op_member(w.V + h.coff[cc] * B, nq, (int64_t)nq * n);
+                    g(OP_N, OP_N, nq, n, nq, op_member(Zc, nq, nn), V, P, nq, nn, 1.0, V, 1.0);  // G W = V + Z V
+                } else {
+                    g(OP_N, OP_N, nq, n, nq, op_member(Gc, nq, nn), W, P, nq, nn);            // G W
+                }
+                g(OP_N, OP_N, n, n, nq, X, op_member(P, nq, nn), Zn, n, nn);                   // Z = X G W
             } else {
                 g(OP_N, OP_N, nq, n, n, W, opGl(sc), P, nq, nn);                               // P = W Gl
+            }
+            // G of this slab: wanted itself, or needed by the next one
+            const int nx2 = sc - step;
+            const bool needG = !zf || full.any || sigma || sc == sf || !zform(nx2) || !kept(nx2) || !w.V;
+            if (!zf)
                 g(OP_N, OP_N, n, n, nq, op_member(GN0, n, nn), op_member(P, nq, nn), Gn, n, nn, 1.0,
                   opGl(sc), 1.0);                                                              // G = Gl + GN0 P
-            }
-            g(OP_N, OP_N, n, nq, nq, op_member(X, n, nn), op_member(Lc, nq, nn), Y, n, nn);    // Y = X G<
-            g(OP_N, OP_C, n, n, nq, op_member(Y, n, nn), op_member(X, n, nn), U, n, nn, 1.0,
-              opGln(sc), 1.0);                                                                 // U = Gln + Y X^H
-            if (!zform || want_j) g(OP_N, OP_N, nq, n, n, W, opGln(sc), Q, nq, nn);           // Q = W Gln
+            else if (needG)
+                g(OP_N, OP_N, n, n, n, op_member(Zn, n, nn), opGl(sc), Gn, n, nn, 1.0, opGl(sc),
+                  1.0);                                                                        // G = Gl + Z Gl
+            g(OP_N, OP_N, n, nq, nq, X, op_member(Lc, nq, nn), Y, n, nn);                      // Y = X G<
+            g(OP_N, OP_C, n, n, nq, op_member(Y, n, nn), X, U, n, nn, 1.0, opGln(sc), 1.0);    // U = Gln + Y X^H
+            if (!zf || want_j || want_gw) g(OP_N, OP_N, nq, n, n, W, opGln(sc), Q, nq, nn);   // Q = W Gln
             if (want_gw) gw_extras(sc, n, W, X, Y, Q, GN0, Gc, Lc, g);
             if (!sigma) {
-                if (zform)
-                    g(OP_N, OP_N, n, n, n, op_member(Z, n, nn), opGln(sc), Y, n, nn);         // Tm = Z Gln
+                if (zf)
+                    g(OP_N, OP_N, n, n, n, op_member(Zn, n, nn), opGln(sc), Y, n, nn);        // Tm = Z Gln
                 else
                     g(OP_N, OP_N, n, n, nq, op_member(GN0, n, nn), op_member(Q, nq, nn), Y, n, nn);  // Tm = GN0 Q
                 // G< = U + Tm - Tm^H: the reference's last term Gln W^H GN0^H equals
@@ -784,15 +834,16 @@ struct Solve {
                 an.Y = op_member(U, n, nn);
                 an.c1 = 1.0;
                 antiherm(s, an);
-            } else {
+            } else if (zf) {
                 // scattering injections (sigma_lesser_ph S, or a Sigma^< that is not
                 // anti-Hermitian) break that symmetry: the reference's four terms
-                if (zform)
-                    g(OP_N, OP_N, n, n, n, op_member(Z, n, nn), opGln(sc), Y, n, nn, 1.0, op_member(U, n, nn),
-                      1.0);                                                                      // U + Z Gln
-                else
-                    g(OP_N, OP_N, n, n, nq, op_member(GN0, n, nn), op_member(Q, nq, nn), Y, n, nn, 1.0,
-                      op_member(U, n, nn), 1.0);                                                 // U + GN0 Q
+                g(OP_N, OP_N, n, n, n, op_member(Zn, n, nn), opGln(sc), Y, n, nn, 1.0, op_member(U, n, nn),
+                  1.0);                                                                          // U + Z Gln
+                g(OP_N, OP_C, n, n, n, opGln(sc), op_member(Zn, n, nn), Ln, n, nn, 1.0, op_member(Y, n, nn),
+                  1.0);                                                                          // + Gln Z^H
+            } else {
+                g(OP_N, OP_N, n, n, nq, op_member(GN0, n, nn), op_member(Q, nq, nn), Y, n, nn, 1.0,
+                  op_member(U, n, nn), 1.0);                                                     // U + GN0 Q
                 g(OP_N, OP_C, n, nq, n, opGln(sc), W, P, n, nn);                                  // Gln W^H
                 g(OP_N, OP_C, n, n, nq, op_member(P, n, nn), op_member(GN0, n, nn), Ln, n, nn, 1.0,
                   op_member(Y, n, nn), 1.0);                                                     // + Gln W^H GN0^H
@@ -800,7 +851,7 @@ struct Solve {
             const double2* jd = nullptr;
             if (want_j) {
                 // A = G<(nbr) X^H + G(nbr) Q ; Jdens = -2 W^H A  (rgf_mod.f90:215-221)
-                g(OP_N, OP_C, nq, n, nq, op_member(Lc, nq, nn), op_member(X, n, nn), U, nq, nn);
+                g(OP_N, OP_C, nq, n, nq, op_member(Lc, nq, nn), X, U, nq, nn);
                 g(OP_N, OP_N, nq, n, nq, op_member(Gc, nq, nn), op_member(Q, nq, nn), U, nq, nn, 1.0,
                   op_member(U, nq, nn), 1.0);
                 g(OP_C, OP_N, n, n, nq, W, op_member(U, nq, nn), T[10], n, nn, -2.0);
@@ -808,7 +859,9 @@ struct Solve {
             }
             std::swap(Gc, Gn);
             std::swap(Lc, Ln);
-            diag_out(sc, Gc, Lc);
+            std::swap(Zc, Zn);
+            haveZ = zf;
+            diag_out(sc, Gc, Lc, zf && !sigma ? Zc : nullptr);
             full_slab(sc, Gc, Lc, jd);
             sn = sc;
         }
@@ -979,6 +1032,18 @@ int qt_ham_create(int32_t nx, const int32_t* nm, int32_t nk, const void* const* 
             if (Sii) same = same && !memcmp(Sii[(int64_t)k * nx], Sii[(int64_t)k * nx + nx - 1], bytes);
         }
         h->leads_same = same;
+        // neighbouring couplings that coincide (every Wannier-built device)
+        h->csame.assign(nx + 1, 0);
+        for (int s = 1; s < nx; ++s) {
+            const int prows = s - 1 < nx ? nm[s - 1] : nm[nx - 1], pcols = s == 1 ? nm[0] : nm[s - 2];
+            bool eq = nm[s] == prows && nm[s - 1] == pcols;
+            for (int k = 0; eq && k < nk; ++k) {
+                const void* a = H1i[(int64_t)k * (nx + 1) + s];
+                const void* b = H1i[(int64_t)k * (nx + 1) + s - 1];
+                eq = a == b || !memcmp(a, b, sizeof(double2) * (size_t)nm[s] * nm[s - 1]);
+            }
+            h->csame[s] = eq;
+        }
         *out = h;
         return QT_OK;
     } catch (const hip_error& e) {
@@ -1003,14 +1068,23 @@ int qt_ham_destroy(qt_ham* h) {
     return QT_OK;
 }
 
-static int choose_batch(qt_ham& h, int npts, bool sigma) {
+// Whether the first pass's coupling products stay resident: where 32 points
+// with them fit the device's memory.  It depends on the device and the shape
+// only, so a point's results do not depend on what else is allocated.
+static bool keep_products(const qt_ham& h, bool sigma) {
+    size_t freeb = 0, total = 0;
+    if (hipMemGetInfo(&freeb, &total) != hipSuccess) return false;
+    return work_bytes(h, 32, sigma, true) <= (size_t)(0.80 * (double)total);
+}
+
+static int choose_batch(qt_ham& h, int npts, bool sigma, bool keep) {
     const char* env = getenv("QT_BATCH");
     if (env && atoi(env) > 0) return std::min(npts, atoi(env));
     size_t freeb = 0, total = 0;
     if (hipMemGetInfo(&freeb, &total) != hipSuccess) freeb = (size_t)8 << 30;
     const size_t budget = (size_t)(0.80 * (double)(freeb + g_ctx->arena.cap));
     int B = std::min(npts, 128);
-    while (B > 1 && work_bytes(h, B, sigma) > budget) B = B * 3 / 4;
+    while (B > 1 && work_bytes(h, B, sigma, keep) > budget) B = B * 3 / 4;
     return std::max(B, 1);
 }
 
@@ -1036,10 +1110,11 @@ int qt_rgf_solve(qt_ham* h, const qt_rgf_params* p, int32_t npts, const double* 
     std::lock_guard<std::mutex> lk(c.mu);
     try {
         QT_HIP(hipSetDevice(c.device));
-        const int B = choose_batch(*h, npts, sigma);
-        c.arena.reserve(work_bytes(*h, B, sigma));
+        const bool keep = keep_products(*h, sigma);
+        const int B = choose_batch(*h, npts, sigma, keep);
+        c.arena.reserve(work_bytes(*h, B, sigma, keep));
         Work w;
-        work_carve(c.arena, w, *h, B, sigma);
+        work_carve(c.arena, w, *h, B, sigma, keep);
         qt_timing tm{};
         tm.batch = B;
         c.timer.reset();
@@ -2396,10 +2471,11 @@ int qt_gw_scba_step(qt_ham* h, const qt_rgf_params* p, int32_t nen, const double
 
         // ---- G of every energy (qt_rgf_solve's batch loop, QT_RGF_GW with sigma)
         {
-            const int B = choose_batch(*h, nen, true);
-            c.arena.reserve(work_bytes(*h, B, true));
+            const bool keep = keep_products(*h, true);
+            const int B = choose_batch(*h, nen, true, keep);
+            c.arena.reserve(work_bytes(*h, B, true, keep));
             Work w;
-            work_carve(c.arena, w, *h, B, true);
+            work_carve(c.arena, w, *h, B, true, keep);
             qt_timing tm{};
             std::vector<double> hz(2 * B), hf(5 * B), htr(B), htre(B);
             std::vector<int> hk(2 * B, 0), hinfo(B);
