@@ -1,9 +1,8 @@
 // qt_gemm.hip -- batched complex128 GEMM on the gfx950 FP64 matrix cores.
 //
-// One workgroup (4 waves, 256 threads) computes a 64x64 complex tile of
-// C = alpha*op(A)op(B) + beta*D for one batch member.  K is staged through
-// LDS in chunks of 16 complex values, double buffered (2 x 32 KB).  Each
-// wave owns a 32x32 sub-tile = 2x2 MFMA tiles of 16x16; a complex product is
+// One workgroup computes a tile of C = alpha*op(A)op(B) + beta*D for one batch
+// member: 32x32 or 64x64 with 4 waves, 128x64 with 4 or 8.  K is staged through
+// LDS in double-buffered chunks.  Each wave owns 16x16 MFMA tiles; a complex product is
 // four v_mfma_f64_16x16x4 (re*re, -im*im into Re; re*im, im*re into Im), or,
 // in the three-multiplication form (G3, QT_PREC_FP64_3M), three:
 //     P1 = Ar Br,  P2 = Ai Bi,  P3 = (Ar + Ai)(Br + Bi)  (sums rounded to FP64),
@@ -36,197 +35,12 @@ namespace qt {
 
 namespace {
 
-constexpr int BM = 64, BN = 64, BK = 16;
+constexpr int BM = 64;
 constexpr int NXCD = 8;
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ double2 cconj(double2 v) { return make_double2(v.x, -v.y); }
-
-template <int OPA, int OPB, bool G3>
-__global__ __launch_bounds__(256, 2) void zgemm_mfma_kernel(ZGemmArgs a, int tiles_m, int tiles,
-                                                            int batch_pad) {
-    // XCD-aware decode: linear id L -> (member, tile), member%8 == L%8
-    const int L = blockIdx.x;
-    const int lane8 = L % NXCD;
-    const int rest = L / NXCD;
-    const int tile = rest % tiles;
-    const int b = lane8 + NXCD * (rest / tiles);
-    if (b >= a.batch) return;
-    if (a.active && !a.active[b]) return;
-    (void)batch_pad;
-
-    const int kz = a.kidx ? a.kidx[b >> a.kshift] : 0;
-    const double2* __restrict__ Ap = a.A.p + b * a.A.sb + kz * a.A.sk;
-    const double2* __restrict__ Bp = a.B.p + b * a.B.sb + kz * a.B.sk;
-    const int64_t lda = a.A.ld, ldb = a.B.ld;
-    const int M = a.M, N = a.N, K = a.K;
-    const int m0 = (tile % tiles_m) * BM;
-    const int n0 = (tile / tiles_m) * BN;
-
-    __shared__ double2 As[2][BK][BM];
-    __shared__ double2 Bs[2][BK][BN];
-
-    const int tid = threadIdx.x;
-    double2 ra[4], rb[4];
-
-    auto loadA = [&](int k0) {
-        if (OPA == OP_N) {
-            const int kk = tid >> 4, ii = (tid & 15) * 4;
-            const int gk = k0 + kk;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int gi = m0 + ii + q;
-                ra[q] = (gi < M && gk < K) ? Ap[gi + gk * lda] : make_double2(0.0, 0.0);
-            }
-        } else {
-            const int ii = tid >> 2, kk = (tid & 3) * 4;
-            const int gi = m0 + ii;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int gk = k0 + kk + q;
-                ra[q] = (gi < M && gk < K) ? Ap[gk + gi * lda] : make_double2(0.0, 0.0);
-            }
-        }
-    };
-    auto storeA = [&](int buf) {
-        if (OPA == OP_N) {
-            const int kk = tid >> 4, ii = (tid & 15) * 4;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) As[buf][kk][ii + q] = ra[q];
-        } else {
-            const int ii = tid >> 2, kk = (tid & 3) * 4;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) As[buf][kk + q][ii] = OPA == OP_C ? cconj(ra[q]) : ra[q];
-        }
-    };
-    auto loadB = [&](int k0) {
-        if (OPB == OP_N) {
-            const int jj = tid >> 2, kk = (tid & 3) * 4;
-            const int gj = n0 + jj;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int gk = k0 + kk + q;
-                rb[q] = (gj < N && gk < K) ? Bp[gk + gj * ldb] : make_double2(0.0, 0.0);
-            }
-        } else {
-            const int kk = tid >> 4, jj = (tid & 15) * 4;
-            const int gk = k0 + kk;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int gj = n0 + jj + q;
-                rb[q] = (gj < N && gk < K) ? Bp[gj + gk * ldb] : make_double2(0.0, 0.0);
-            }
-        }
-    };
-    auto storeB = [&](int buf) {
-        if (OPB == OP_N) {
-            const int jj = tid >> 2, kk = (tid & 3) * 4;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) Bs[buf][kk + q][jj] = rb[q];
-        } else {
-            const int kk = tid >> 4, jj = (tid & 15) * 4;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) Bs[buf][kk][jj + q] = OPB == OP_C ? cconj(rb[q]) : rb[q];
-        }
-    };
-
-    const int wave = tid >> 6, lane = tid & 63;
-    const int wm = wave & 1, wn = wave >> 1;
-    const int li = lane & 15, lk = lane >> 4;
-
-    // G3: accR = P1, accI = P2, acc3 = P3
-    double4_t accR[2][2], accI[2][2], acc3[G3 ? 2 : 1][G3 ? 2 : 1];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            accR[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
-            accI[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
-            if constexpr (G3) acc3[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
-        }
-
-    const int nk = (K + BK - 1) / BK;
-    loadA(0);
-    loadB(0);
-    storeA(0);
-    storeB(0);
-    __syncthreads();
-
-    for (int kt = 0; kt < nk; ++kt) {
-        const int buf = kt & 1;
-        if (kt + 1 < nk) {
-            loadA((kt + 1) * BK);
-            loadB((kt + 1) * BK);
-        }
-#pragma unroll
-        for (int kq = 0; kq < BK / 4; ++kq) {
-            const int k = kq * 4 + lk;
-            double2 av[2], bv[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) av[i] = As[buf][k][wm * 32 + i * 16 + li];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) bv[j] = Bs[buf][k][wn * 32 + j * 16 + li];
-            if constexpr (G3) {
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j].x, av[i].x, accR[i][j], 0, 0, 0);
-                        accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j].y, av[i].y, accI[i][j], 0, 0, 0);
-                        acc3[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j].x + bv[j].y, av[i].x + av[i].y,
-                                                                         acc3[i][j], 0, 0, 0);
-                    }
-            } else {
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j].x, av[i].x, accR[i][j], 0, 0, 0);
-                        accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(-bv[j].y, av[i].y, accR[i][j], 0, 0, 0);
-                        accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j].y, av[i].x, accI[i][j], 0, 0, 0);
-                        accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j].x, av[i].y, accI[i][j], 0, 0, 0);
-                    }
-            }
-        }
-        if (kt + 1 < nk) {
-            storeA(buf ^ 1);
-            storeB(buf ^ 1);
-        }
-        __syncthreads();
-    }
-
-    // epilogue
-    double2* __restrict__ Cp = a.C + b * a.sbc + kz * a.skc;
-    const double2* __restrict__ Dp = a.D.p ? a.D.p + b * a.D.sb + kz * a.D.sk : nullptr;
-    const double alpha = a.alpha, beta = a.beta;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int gi = m0 + wm * 32 + i * 16 + li;
-        if (gi >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int gj = n0 + wn * 32 + j * 16 + 4 * q + lk;
-                if (gj >= N || (gj >= a.skip_lo && gj < a.skip_hi)) continue;
-                double cr = accR[i][j][q], ci = accI[i][j][q];
-                if constexpr (G3) {
-                    const double p1 = accR[i][j][q], p2 = accI[i][j][q];
-                    cr = p1 - p2;
-                    ci = (acc3[i][j][q] - p1) - p2;
-                }
-                double re = alpha * cr, im = alpha * ci;
-                if (Dp) {
-                    const double2 d = Dp[gi + gj * a.D.ld];
-                    re += beta * d.x;
-                    im += beta * d.y;
-                }
-                Cp[gi + gj * a.ldc] = make_double2(re, im);
-            }
-        }
-    }
-}
 
 // Wider variant: 128x64 block tile, K staged 8 at a time (2 x 24 KB LDS),
 // each wave a 64x32 sub-tile (4x2 MFMA tiles): twice the MFMAs per LDS read
@@ -435,7 +249,7 @@ __global__ __launch_bounds__(256, 2) void zgemm_mfma_wide_kernel(ZGemmArgs a, in
 }
 
 // 128x64 tiles with 8 waves of 32x32 (2x2 MFMA tiles each): the 128x64
-// kernel's LDS staging and global loads, the 64x64 kernel's per-wave register
+// kernel's LDS staging and global loads, the 64x64 tile's per-wave register
 // tile, so the accumulators of the three-multiplication form fit beside
 // more waves per CU.  Every output element sees the MFMAs of the other two
 // kernels in the same order.
@@ -601,6 +415,183 @@ __global__ __launch_bounds__(512, G3 ? 1 : 2) void zgemm_mfma_w8_kernel(ZGemmArg
     }
 }
 
+// 32x32 and 64x64 tiles: WGM x WGN waves of TM x TN MFMA tiles, K staged KB at a
+// time in two LDS buffers with rows padded by one element (lanes along k then
+// write distinct banks).  Every output element sees the MFMAs of the other
+// kernels in the same order.
+//
+// 64x64 staged 8 deep: 33 KB of LDS and 125 registers, so four workgroups a CU
+// where a 16-deep stage took two; 16 members of 695^3 0.785 -> 0.715 ms, 48 of
+// 250^3 0.127 -> 0.115.  32x32 for blocks of a few hundred orbitals and less,
+// where 64-row tiles leave the chip short of workgroups (64^3 x 256 members is one
+// a CU, 192^3 x 60 is 540 for 512 places) or compute padding (160 = 2.5 x 64):
+// 100 of 160^3 0.098 -> 0.068 ms, 60 of 192^3 0.095 -> 0.072, 16 of 128^3
+// 0.027 -> 0.013, 256 of 96^3 0.057 (128x64) -> 0.041, 16 of 591x195x591 0.299
+// (128x64) -> 0.191, one of 32^3 10.6 -> 6.5 us.  Half the operand reuse makes it
+// L2 bound, the slower one, once both sides are above 384.  Staged 16 deep it
+// is 1-5% faster where K is below a hundred (fewer barriers), 8 deep (17 KB, up
+// to eight workgroups a CU) 3-5% above.
+template <int OPA, int OPB, bool G3, int TM, int TN, int WGM, int WGN, int KB>
+__global__ __launch_bounds__(WGM * WGN * 64)
+    __attribute__((amdgpu_waves_per_eu(G3 ? (TM * TN == 4 ? 2 : 4) : 4))) void zgemm_mfma_small_kernel(ZGemmArgs a,
+                                                                                                      int tiles_m,
+                                                                                                      int tiles) {
+    constexpr int SM = TM * WGM * 16, SN = TN * WGN * 16, NT = WGM * WGN * 64;
+    constexpr int QA = SM * KB / NT, QB = SN * KB / NT;
+    static_assert(SM * KB % NT == 0 && SN * KB % NT == 0, "whole loads");
+    const int L = blockIdx.x;
+    const int lane8 = L % NXCD;
+    const int rest = L / NXCD;
+    const int tile = rest % tiles;
+    const int b = lane8 + NXCD * (rest / tiles);
+    if (b >= a.batch) return;
+    if (a.active && !a.active[b]) return;
+
+    const int kz = a.kidx ? a.kidx[b >> a.kshift] : 0;
+    const double2* __restrict__ Ap = a.A.p + b * a.A.sb + kz * a.A.sk;
+    const double2* __restrict__ Bp = a.B.p + b * a.B.sb + kz * a.B.sk;
+    const int64_t lda = a.A.ld, ldb = a.B.ld;
+    const int M = a.M, N = a.N, K = a.K;
+    const int m0 = (tile % tiles_m) * SM;
+    const int n0 = (tile / tiles_m) * SN;
+
+    __shared__ double2 As[2][KB][SM + 1];
+    __shared__ double2 Bs[2][KB][SN + 1];
+
+    const int tid = threadIdx.x;
+    double2 ra[QA], rb[QB];
+    // element e = tid + NT q of a stage: along the memory's contiguous axis
+    auto loadA = [&](int k0) {
+#pragma unroll
+        for (int q = 0; q < QA; ++q) {
+            const int e = tid + NT * q;
+            const int ii = OPA == OP_N ? e % SM : e / KB, kk = OPA == OP_N ? e / SM : e % KB;
+            const int gi = m0 + ii, gk = k0 + kk;
+            ra[q] = (gi < M && gk < K) ? (OPA == OP_N ? Ap[gi + gk * lda] : Ap[gk + gi * lda])
+                                       : make_double2(0.0, 0.0);
+        }
+    };
+    auto loadB = [&](int k0) {
+#pragma unroll
+        for (int q = 0; q < QB; ++q) {
+            const int e = tid + NT * q;
+            const int jj = OPB == OP_N ? e / KB : e % SN, kk = OPB == OP_N ? e % KB : e / SN;
+            const int gj = n0 + jj, gk = k0 + kk;
+            rb[q] = (gj < N && gk < K) ? (OPB == OP_N ? Bp[gk + gj * ldb] : Bp[gj + gk * ldb])
+                                       : make_double2(0.0, 0.0);
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int q = 0; q < QA; ++q) {
+            const int e = tid + NT * q;
+            const int ii = OPA == OP_N ? e % SM : e / KB, kk = OPA == OP_N ? e / SM : e % KB;
+            As[buf][kk][ii] = OPA == OP_C ? cconj(ra[q]) : ra[q];
+        }
+#pragma unroll
+        for (int q = 0; q < QB; ++q) {
+            const int e = tid + NT * q;
+            const int jj = OPB == OP_N ? e / KB : e % SN, kk = OPB == OP_N ? e % KB : e / SN;
+            Bs[buf][kk][jj] = OPB == OP_C ? cconj(rb[q]) : rb[q];
+        }
+    };
+
+    const int wave = tid >> 6, lane = tid & 63;
+    const int wm = wave % WGM, wn = wave / WGM;
+    const int li = lane & 15, lk = lane >> 4;
+
+    double4_t accR[TM][TN], accI[TM][TN], acc3[G3 ? TM : 1][G3 ? TN : 1];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            accR[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
+            accI[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
+            if constexpr (G3) acc3[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
+        }
+
+    const int nk = (K + KB - 1) / KB;
+    loadA(0);
+    loadB(0);
+    store(0);
+    __syncthreads();
+    for (int kt = 0; kt < nk; ++kt) {
+        const int buf = kt & 1;
+        if (kt + 1 < nk) {
+            loadA((kt + 1) * KB);
+            loadB((kt + 1) * KB);
+        }
+#pragma unroll
+        for (int kq = 0; kq < KB / 4; ++kq) {
+            const int k = kq * 4 + lk;
+            double2 av[TM], bv[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) av[i] = As[buf][k][(wm * TM + i) * 16 + li];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) bv[j] = Bs[buf][k][(wn * TN + j) * 16 + li];
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j].x, av[i].x, accR[i][j], 0, 0, 0);
+                    if constexpr (G3) {
+                        accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j].y, av[i].y, accI[i][j], 0, 0, 0);
+                        acc3[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j].x + bv[j].y, av[i].x + av[i].y,
+                                                                         acc3[i][j], 0, 0, 0);
+                    } else {
+                        accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j].y, av[i].x, accI[i][j], 0, 0, 0);
+                        accR[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(-bv[j].y, av[i].y, accR[i][j], 0, 0, 0);
+                        accI[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j].x, av[i].y, accI[i][j], 0, 0, 0);
+                    }
+                }
+        }
+        if (kt + 1 < nk) store(buf ^ 1);
+        __syncthreads();
+    }
+
+    double2* __restrict__ Cp = a.C + b * a.sbc + kz * a.skc;
+    const double2* __restrict__ Dp = a.D.p ? a.D.p + b * a.D.sb + kz * a.D.sk : nullptr;
+    const double alpha = a.alpha, beta = a.beta;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int gi = m0 + (wm * TM + i) * 16 + li;
+        if (gi >= M) continue;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int gj = n0 + (wn * TN + j) * 16 + 4 * q + lk;
+                if (gj >= N || (gj >= a.skip_lo && gj < a.skip_hi)) continue;
+                double cr = accR[i][j][q], ci = accI[i][j][q];
+                if constexpr (G3) {
+                    const double p1 = accR[i][j][q], p2 = accI[i][j][q];
+                    cr = p1 - p2;
+                    ci = (acc3[i][j][q] - p1) - p2;
+                }
+                double re = alpha * cr, im = alpha * ci;
+                if (Dp) {
+                    const double2 d = Dp[gi + gj * a.D.ld];
+                    re += beta * d.x;
+                    im += beta * d.y;
+                }
+                Cp[gi + gj * a.ldc] = make_double2(re, im);
+            }
+        }
+    }
+}
+
+template <int OPA, int OPB, bool G3, int TM, int TN, int WGM, int WGN, int KB>
+void launch_small(hipStream_t s, const ZGemmArgs& a) {
+    constexpr int SM = TM * WGM * 16, SN = TN * WGN * 16;
+    const int tiles_m = (a.M + SM - 1) / SM;
+    const int tiles = tiles_m * ((a.N + SN - 1) / SN);
+    const int64_t blocks = (int64_t)tiles * ((a.batch + NXCD - 1) / NXCD * NXCD);
+    if (blocks > 0x7fffffff) throw hip_error("zgemm: grid too large", 1);
+    hipLaunchKernelGGL((zgemm_mfma_small_kernel<OPA, OPB, G3, TM, TN, WGM, WGN, KB>), dim3((unsigned)blocks),
+                       dim3(WGM * WGN * 64), 0, s, a, tiles_m, tiles);
+    QT_HIP(hipGetLastError());
+}
+
 template <int OPA, int OPB, bool G3>
 void launch_w8(hipStream_t s, const ZGemmArgs& a) {
     const int tiles_m = (a.M + WBM - 1) / WBM;
@@ -627,19 +618,23 @@ void launch_wide(hipStream_t s, const ZGemmArgs& a) {
     QT_HIP(hipGetLastError());
 }
 
-// Tile choice.  QT_GEMM_TILE=64x64, =128x64 or =128x64w8 fixes the kernel;
+// Tile choice.  QT_GEMM_TILE=64x64, 128x64, 128x64w8, 32x32 or 32x32k8 fixes the
+// kernel;
 // otherwise the autotuner below picks per shape (QT_GEMM_TUNE=0: the
-// row-waste rule of use_wide alone).  All three kernels accumulate every
+// row-waste rule of use_wide alone).  All kernels accumulate every
 // output element in the same order (k ascending in groups of 4, the same
 // MFMAs per group and component, the same epilogue), so the choice never
 // changes a result.
-enum { TILE_AUTO = 0, TILE_NARROW = 1, TILE_WIDE = 2, TILE_W8 = 3 };
+enum { TILE_AUTO = 0, TILE_NARROW = 1, TILE_WIDE = 2, TILE_W8 = 3, TILE_32X32 = 4, TILE_32K8 = 5, NTILE = 5 };
+const char* tile_name(int t) {
+    static const char* const n[] = {"auto", "64x64", "128x64", "128x64w8", "32x32", "32x32k8"};
+    return n[t];
+}
 int tile_forced() {
     static const int v = [] {
         const char* e = getenv("QT_GEMM_TILE");
-        if (e && std::string(e) == "64x64") return (int)TILE_NARROW;
-        if (e && std::string(e) == "128x64") return (int)TILE_WIDE;
-        if (e && std::string(e) == "128x64w8") return (int)TILE_W8;
+        for (int t = 1; e && t <= NTILE; ++t)
+            if (std::string(e) == tile_name(t)) return t;
         return (int)TILE_AUTO;
     }();
     return v;
@@ -665,21 +660,8 @@ bool use_wide(int M) {
     return M >= WBM && waste_wide <= waste_narrow;
 }
 
-template <int OPA, int OPB, bool G3>
-void launch_narrow(hipStream_t s, const ZGemmArgs& a) {
-    const int tiles_m = (a.M + BM - 1) / BM;
-    const int tiles_n = (a.N + BN - 1) / BN;
-    const int tiles = tiles_m * tiles_n;
-    const int batch_pad = (a.batch + NXCD - 1) / NXCD * NXCD;
-    const int64_t blocks = (int64_t)tiles * batch_pad;
-    if (blocks > 0x7fffffff) throw hip_error("zgemm: grid too large", 1);
-    hipLaunchKernelGGL((zgemm_mfma_kernel<OPA, OPB, G3>), dim3((unsigned)blocks), dim3(256), 0, s, a,
-                       tiles_m, tiles, batch_pad);
-    QT_HIP(hipGetLastError());
-}
-
 // Autotuner: the first product of each shape (op pair, M, N, K, batch) runs
-// the three kernels twice into a scratch output (the operands and the addend are
+// the kernels in question twice into a scratch output (the operands and the addend are
 // only read; at most 512 MiB of scratch, fewer members where the full batch
 // needs more) after the work already queued on the stream, and the faster
 // kernel is kept for the shape for the life of the process.  Where the
@@ -695,12 +677,27 @@ TuneState& tune_state() {
 
 template <int OPA, int OPB, bool G3>
 void launch_tile(hipStream_t s, const ZGemmArgs& a, int tile) {
-    if (tile == TILE_W8)
+    if (tile == TILE_32X32)
+        launch_small<OPA, OPB, G3, 1, 1, 2, 2, 16>(s, a);
+    else if (tile == TILE_32K8)
+        launch_small<OPA, OPB, G3, 1, 1, 2, 2, 8>(s, a);
+    else if (tile == TILE_W8)
         launch_w8<OPA, OPB, G3>(s, a);
     else if (tile == TILE_WIDE)
         launch_wide<OPA, OPB, G3>(s, a);
     else
-        launch_narrow<OPA, OPB, G3>(s, a);
+        launch_small<OPA, OPB, G3, 2, 2, 2, 2, 8>(s, a);
+}
+
+// the kernels worth timing for an M x N output: 32x32 tiles where one side is up
+// to 384 (above, 64-row tiles fill the chip and need half the operand traffic),
+// 128-row ones where more than half of such a tile is used
+bool in_question(int tile, int M, int N) {
+    switch (tile) {
+        case TILE_WIDE: case TILE_W8: return M > 64;
+        case TILE_32X32: case TILE_32K8: return std::min(M, N) <= 384;
+        default: return true;
+    }
 }
 
 template <int OPA, int OPB, bool G3>
@@ -723,7 +720,8 @@ int tuned_tile(hipStream_t s, const ZGemmArgs& a) {
     t.skip_lo = t.skip_hi = 0;
     void* scratch = nullptr;
     hipEvent_t ev[3];
-    float ms[3] = {1e30f, 1e30f, 1e30f};  // 64x64, 128x64, 128x64 with 8 waves
+    float ms[NTILE + 1];
+    for (float& m : ms) m = 1e30f;
     if (hipMalloc(&scratch, per * (size_t)members) != hipSuccess) {
         (void)hipGetLastError();  // no room for the scratch output: the row-waste rule, kept
         const int tile = use_wide(a.M) ? TILE_WIDE : TILE_NARROW;
@@ -734,9 +732,10 @@ int tuned_tile(hipStream_t s, const ZGemmArgs& a) {
     for (auto& e : ev) QT_HIP(hipEventCreate(&e));
     t.C = (double2*)scratch;
     for (int rep = 0; rep < 2; ++rep)
-        for (int v = 0; v < 3; ++v) {
+        for (int v = 1; v <= NTILE; ++v) {
+            if (!in_question(v, a.M, a.N)) continue;
             QT_HIP(hipEventRecord(ev[0], s));
-            launch_tile<OPA, OPB, G3>(s, t, v + 1);
+            launch_tile<OPA, OPB, G3>(s, t, v);
             QT_HIP(hipEventRecord(ev[1], s));
             QT_HIP(hipEventSynchronize(ev[1]));
             float m = 0.0f;
@@ -745,16 +744,16 @@ int tuned_tile(hipStream_t s, const ZGemmArgs& a) {
         }
     for (auto& e : ev) QT_HIP(hipEventDestroy(e));
     QT_HIP(hipFree(scratch));
-    int best = 0;
-    for (int v = 1; v < 3; ++v)
-        if (ms[v] < ms[best]) best = v;
-    const int tile = best + 1;
-    if (tune_log())
-        fprintf(stderr,
-                "qt gemm tune: ops %d%s M %d N %d K %d batch %d (%d timed): 64x64 %.4f ms, 128x64 %.4f ms, "
-                "128x64w8 %.4f ms -> %s\n",
-                OPA * 3 + OPB, G3 ? " (3m)" : "", a.M, a.N, a.K, a.batch, members, ms[0], ms[1], ms[2],
-                tile == TILE_W8 ? "128x64w8" : (tile == TILE_WIDE ? "128x64" : "64x64"));
+    int tile = TILE_NARROW;
+    for (int v = 1; v <= NTILE; ++v)
+        if (ms[v] < ms[tile]) tile = v;
+    if (tune_log()) {
+        fprintf(stderr, "qt gemm tune: ops %d%s M %d N %d K %d batch %d (%d timed):", OPA * 3 + OPB, G3 ? " (3m)" : "",
+                a.M, a.N, a.K, a.batch, members);
+        for (int v = 1; v <= NTILE; ++v)
+            if (ms[v] < 1e30f) fprintf(stderr, " %s %.4f ms", tile_name(v), ms[v]);
+        fprintf(stderr, " -> %s\n", tile_name(tile));
+    }
     std::lock_guard<std::mutex> lk(ts.mu);
     ts.tile[key] = tile;
     return tile;
