@@ -182,7 +182,7 @@ struct Work {
 size_t work_bytes(const qt_ham& h, int B, bool sigma, bool keep = false);
 void work_carve(Arena& a, Work& w, const qt_ham& h, int B, bool sigma, bool keep = false);
 void inv_batch(Ctx& c, Work& w, int n, int batch, double2* A, int64_t sa, double2* X, int64_t sx,
-               const int* active, int flop_batch = -1);
+               const int* active, int flop_batch = -1, bool lookahead = true);
 void note_inv_info(Ctx& c, Work& w, int batch, int period);
 
 // ------------------------------------------------------------ Sancho-Rubio
@@ -211,6 +211,13 @@ struct SanchoIO {
     int period = 1;               // member m belongs to point m % period
     int64_t total_iters = 0;      // host: sum of iterations over members
 };
+
+// The decimation doubles its chain every step and its rounding errors grow like
+// 1 / eta^2 next to band edges: below this broadening two correct operation
+// orders of the inversion part the contact currents by 1e-10 (median of 60
+// devices of 160 orbitals at eta = 1e-5) to 1e-6, so there it keeps the panel and
+// update kernels whose results the parity classification was measured on.
+constexpr double kLookaheadEta = 1e-4;
 
 void sancho_run(Ctx& c, Work& w, SanchoIO& io);
 

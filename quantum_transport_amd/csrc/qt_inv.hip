@@ -28,6 +28,9 @@
 //      other rows were eliminated with, which is what gives Gauss-Jordan its
 //      small residual |A X - I|; multiplying by the panel's explicit
 //      inv(A_KK) instead loses up to cond(A_KK) of it.
+// Blocks of 65 to 384 take, where the caller allows it (InvArgs::lookahead), one
+// launch per panel instead (gj_step_kernel): the panel's workgroups bring their
+// columns up to date and factor them while others replay the panel before.
 // Blocks of n <= 64 are inverted by one kernel holding the whole matrix in
 // registers (gj_small_kernel: the same pivot rule and row operations, no
 // panel records).
@@ -357,6 +360,553 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void gj
     }
 }
 
+// ------------------------------------------------------------ look-ahead steps
+constexpr int kLaNB = 32;   // panel and tile width
+constexpr int kLaMax = 384;  // largest block: six waves of 64 rows
+
+template <int CTRL>
+__device__ __forceinline__ double dpp_rotate(double x) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), CTRL, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+// maximum over each 16-lane row, in every lane (rotations by 8, 4, 2, 1)
+__device__ __forceinline__ double row16_max(double x) {
+    x = fmax(x, dpp_rotate<0x128>(x));
+    x = fmax(x, dpp_rotate<0x124>(x));
+    x = fmax(x, dpp_rotate<0x122>(x));
+    return fmax(x, dpp_rotate<0x121>(x));
+}
+
+// 1 / (a.x + i a.y) with one reciprocal, refined by two Newton steps (the
+// hardware seed has more than 20 correct bits), of |a|^2; operands whose
+// squares would leave the normal range are scaled by a power of two first.
+// (Smith's form takes three dependent divisions.)  a is uniform over the wave.
+__device__ __forceinline__ double2 crecip_fast(double2 a) {
+    double t = fma(a.x, a.x, a.y * a.y);
+    int e = 0;
+    if (!(t > 1e-280 && t < 1e280)) {
+        e = __builtin_amdgcn_frexp_exp(fmax(fabs(a.x), fabs(a.y)));
+        a.x = ldexp(a.x, -e);
+        a.y = ldexp(a.y, -e);
+        t = fma(a.x, a.x, a.y * a.y);
+    }
+    double r = __builtin_amdgcn_rcp(t);
+    r = fma(r, fma(-t, r, 1.0), r);
+    r = fma(r, fma(-t, r, 1.0), r);
+    a.x *= r;
+    a.y *= -r;
+    if (e != 0) {
+        a.x = ldexp(a.x, -e);
+        a.y = ldexp(a.y, -e);
+    }
+    return a;
+}
+
+// Replays the NB row operations of the panel at kb (w columns of it) on tile
+// columns [c0, c0 + NB): y by forward substitution of the pivot rows with the
+// multipliers they received before their own step, into Ys (rows beyond w and
+// columns beyond n are zero).  16 lanes per column hold the values of pivot
+// rows ta and ta + 16; y_c is broadcast by a lane shuffle, no barrier.
+template <int NB, int NW>
+__device__ __forceinline__ void solve_y(const double2* Ab, const double2* Gb, const int* pv, int n, int kb, int w,
+                                        int c0, double2 (*Lk)[NB + 1], double2 (*Ys)[NB + 1], double2* dprev,
+                                        signed char* pos) {
+    constexpr int NT = NW * 64, H = NB / 16, CP = (NB / 4 + NW - 1) / NW;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    for (int r = tid; r < n; r += NT) pos[r] = -1;
+    for (int e = tid; e < NB * NB; e += NT) {
+        const int t = e / NB, c = e % NB;
+        Lk[t][c] = (t < w && c < t) ? Gb[(unsigned)(c * n + pv[kb + t])] : make_double2(0.0, 0.0);
+    }
+    if (tid < w) dprev[tid] = Gb[(unsigned)(tid * n + pv[kb + tid])];
+    const int ta = lane & 15, src0 = lane & ~15;
+    double2 y[CP][H];
+#pragma unroll
+    for (int m = 0; m < CP; ++m) {
+        const int cc = (m * NW + wave) * 4 + (lane >> 4), col = c0 + cc;
+#pragma unroll
+        for (int h = 0; h < H; ++h)
+            y[m][h] = (cc < NB && col < n && ta + 16 * h < w) ? Ab[(unsigned)(pv[kb + ta + 16 * h] + col * n)]
+                                                               : make_double2(0.0, 0.0);
+    }
+    __syncthreads();
+    if (tid < w) pos[pv[kb + tid]] = (signed char)tid;
+#pragma unroll
+    for (int ch = 0; ch < H; ++ch) {
+        for (int cl = 0; cl < 16; ++cl) {
+            const int c = 16 * ch + cl;
+            double2 l[H];
+#pragma unroll
+            for (int h = 0; h < H; ++h) l[h] = Lk[ta + 16 * h][c];  // zero up to its own step
+#pragma unroll
+            for (int m = 0; m < CP; ++m) {
+                double2 yc;
+                yc.x = __shfl(y[m][ch].x, src0 + cl, 64);
+                yc.y = __shfl(y[m][ch].y, src0 + cl, 64);
+#pragma unroll
+                for (int h = ch; h < H; ++h) {
+                    y[m][h].x = fma(-l[h].x, yc.x, y[m][h].x);
+                    y[m][h].x = fma(l[h].y, yc.y, y[m][h].x);
+                    y[m][h].y = fma(-l[h].x, yc.y, y[m][h].y);
+                    y[m][h].y = fma(-l[h].y, yc.x, y[m][h].y);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < CP; ++m) {
+        const int cc = (m * NW + wave) * 4 + (lane >> 4);
+        if (cc < NB) {
+#pragma unroll
+            for (int h = 0; h < H; ++h) Ys[ta + 16 * h][cc] = y[m][h];
+        }
+    }
+    __syncthreads();
+}
+
+// acc (one 16-row block, its columns in the matrix layout) <- acc - G y; a
+// pivot row starts from its y, takes the later steps only and is multiplied by
+// 1 / pivot.
+template <int NB>
+__device__ __forceinline__ void replay_block(const double2* Gb, int n, int w, int row, int li, int lk,
+                                             const double2 (*Ys)[NB + 1], const double2* dprev,
+                                             const signed char* pos, double4_t* accR, double4_t* accI) {
+    constexpr int KS = NB / 4, NTL = NB / 16;
+    const bool rok = row < n;
+    double2 g[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        const int k = ks * 4 + lk;
+        g[ks] = (rok && k < w) ? Gb[(unsigned)(k * n + row)] : make_double2(0.0, 0.0);
+    }
+    const int st = rok ? pos[row] : -1;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        const bool keep = ks * 4 + lk > st;
+        g[ks].x = keep ? g[ks].x : 0.0;
+        g[ks].y = keep ? g[ks].y : 0.0;
+    }
+    if (st >= 0) {
+#pragma unroll
+        for (int t = 0; t < NTL; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const double2 y = Ys[st][16 * t + 4 * q + lk];
+                accR[t][q] = y.x;
+                accI[t][q] = y.y;
+            }
+    }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+        for (int t = 0; t < NTL; ++t) {
+            const double2 y = Ys[ks * 4 + lk][16 * t + li];
+            accR[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-y.x, g[ks].x, accR[t], 0, 0, 0);
+            accI[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-y.y, g[ks].x, accI[t], 0, 0, 0);
+            accR[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(y.y, g[ks].y, accR[t], 0, 0, 0);
+            accI[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-y.x, g[ks].y, accI[t], 0, 0, 0);
+        }
+    }
+    if (st >= 0) {
+        const double2 d = dprev[st];
+#pragma unroll
+        for (int t = 0; t < NTL; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const double2 v = cmul(make_double2(accR[t][q], accI[t][q]), d);
+                accR[t][q] = v.x;
+                accI[t][q] = v.y;
+            }
+    }
+}
+
+// One step of the inversion.  The first gridDim.x - nupd workgroups (one per
+// member, padded to a multiple of 8) bring the panel at kb up to date with the
+// previous panel's operations and factor it; the others replay the previous
+// panel (kprev) on one NB-column tile each, all but that panel and the one at
+// kb.  So the factorisation, a latency-bound chain of one workgroup per member,
+// runs beside the matrix work of the step before it in one launch, instead of
+// the two alternating.  Workgroup ids go round-robin over the 8 XCDs: a member's
+// tiles stay on the XCD of its panel.
+//
+// The panel: wave w holds rows 64 w .. 64 w + 63 as four blocks of 16 in the
+// layout of v_mfma_f64_16x16x4; lane (li, lk) = (lane % 16, lane / 16) holds row li
+// of a block and columns 4 q + lk of its 16-column tile t, so the four columns
+// of group g = 4 t + q are the four lane quarters of one register.  A group's
+// four steps run with one row per lane, its four columns turned around through
+// LDS: each 16-lane row finds its candidate key (value and row in one double)
+// and publishes it with that row's four entries, one barrier, and every wave
+// takes the largest key and the pivot row's entries.  The panel's other columns
+// then see the four steps at once,
+//   y_t = a_{p_t} - sum_{c < t} g_{p_t,c} y_c,   a_r <- a_r - sum_c g_rc y_c,
+// on the matrix cores, y solved by every wave for itself from the raw pivot
+// rows in LDS; a pivot row starts from its own y and takes the later steps, the
+// row operations of the unblocked elimination in their order.
+//
+// Bound by the panel's chain: some 1400 cycles a column (search, barrier,
+// reciprocal, update) and 5900 a group for turning and matrix work.  One
+// stream: 48 members of 250 0.888 -> 0.731 ms, 60 of 192 0.645 -> 0.559, 32 of
+// 384 1.55 -> 1.29, 48 of 300 1.24 -> 1.07; at 512 the two are level (the panel's
+// eight waves share the matrix cores of one CU), so the line lies at 384.
+template <int NW>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void gj_step_kernel(
+    double2* A, int64_t sa, const double2* Gprev, double2* Gm, int64_t sg, int n, int batch, int npan, int ntiles,
+    int kprev, int kb, int* pivp, int* info, const int* active) {
+    constexpr int NB = kLaNB, R = 1, NT = NW * 64, NTL = NB / 16, NG = NB / 4, RB = 4 * R, NR = NW * R * 64;
+    static_assert(NW <= 8, "at most 32 row groups");
+    // LDS: the replay's arrays are dead once the panel is factored
+    struct Replay {
+        double2 L[NB][NB + 1], Y[NB][NB + 1], d[NB];
+        signed char pos[1024];
+    };
+    struct Panel {
+        double2 crow[2][32][4];     // entries of each 16-lane row's candidate in the group's columns
+        double2 lrow[2][4][4];      // by group parity: multipliers of the group's pivot rows
+        double2 raw[2][4][NB];      // the group's pivot rows before the group
+        double2 yb[2][4][NB];       // their values when they were eliminated with
+        double2 dfac[NB];           // 1 / pivot of step c
+        double2 gx[4][NR];          // the group's columns / multipliers between the two layouts
+        double cand[2][32];         // candidate key of each 16-lane row, by step parity
+        int pcol[NB];               // pivot row of step c
+    };
+    __shared__ union {
+        Replay r;
+        Panel p;
+    } sm;
+    __shared__ unsigned used[32];   // rows pivoted before this panel (n <= 1024)
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int li = lane & 15, lk = lane >> 4;
+    const int row0 = wave * R * 64;  // the wave's first row
+    const int wprev = kprev >= 0 ? min(NB, n - kprev) : 0;
+
+    if ((int)blockIdx.x >= npan) {  // ---- replay on one tile
+        const int lin = blockIdx.x - npan;
+        const int b = ((lin >> 3) / ntiles) * 8 + (lin & 7);
+        const int c0 = ((lin >> 3) % ntiles) * NB;
+        if (b >= batch || (active && !active[b]) || c0 == kprev || c0 == kb) return;
+        double2* Ab = A + b * sa;
+        const double2* Gp = Gprev + b * sg;
+        solve_y<NB, NW>(Ab, Gp, pivp + (int64_t)b * n, n, kprev, wprev, c0, sm.r.L, sm.r.Y, sm.r.d, sm.r.pos);
+#pragma unroll 1
+        for (int i = 0; i < RB; ++i) {
+            const int row = (i * NW + wave) * 16 + li;  // blocks dealt over the waves
+            if ((i * NW + wave) * 16 >= n) break;
+            double4_t aR[NTL], aI[NTL];
+#pragma unroll
+            for (int t = 0; t < NTL; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int col = c0 + 16 * t + 4 * q + lk;
+                    const double2 v = (row < n && col < n) ? Ab[(unsigned)(row + col * n)] : make_double2(0.0, 0.0);
+                    aR[t][q] = v.x;
+                    aI[t][q] = v.y;
+                }
+            replay_block<NB>(Gp, n, wprev, row, li, lk, sm.r.Y, sm.r.d, sm.r.pos, aR, aI);
+            if (row >= n) continue;
+#pragma unroll
+            for (int t = 0; t < NTL; ++t)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int col = c0 + 16 * t + 4 * q + lk;
+                    if (col < n) Ab[(unsigned)(row + col * n)] = make_double2(aR[t][q], aI[t][q]);
+                }
+        }
+        return;
+    }
+
+    // ---- the panel at kb
+    const int b = blockIdx.x;
+    if (b >= batch || (active && !active[b])) return;
+    double2* Ab = A + b * sa;
+    double2* Gb = Gm + b * sg;             // multiplier of row r at step c: Gb[c*n + r]
+    int* pv = pivp + (int64_t)b * n;
+    const int ncols = min(NB, n - kb);
+
+    if (tid < 32) used[tid] = 0u;
+    __syncthreads();
+    for (int j = tid; j < kb; j += NT) atomicOr(&used[(pv[j] >> 5) & 31], 1u << (pv[j] & 31));
+
+    // offsets are 32-bit: n <= 1024
+    double4_t accR[RB][NTL], accI[RB][NTL];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+        const int row = row0 + i * 16 + li;
+#pragma unroll
+        for (int t = 0; t < NTL; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int col = 16 * t + 4 * q + lk;
+                const double2 v = (row < n && col < ncols) ? Ab[(unsigned)(row + (kb + col) * n)]
+                                                           : make_double2(0.0, 0.0);
+                accR[i][t][q] = v.x;
+                accI[i][t][q] = v.y;
+            }
+    }
+    if (kprev >= 0) {
+        const double2* Gp = Gprev + b * sg;
+        solve_y<NB, NW>(Ab, Gp, pv, n, kprev, wprev, kb, sm.r.L, sm.r.Y, sm.r.d, sm.r.pos);
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+            replay_block<NB>(Gp, n, wprev, row0 + i * 16 + li, li, lk, sm.r.Y, sm.r.d, sm.r.pos, accR[i], accI[i]);
+        __syncthreads();  // the replay's LDS is free
+    }
+    auto& cand = sm.p.cand;
+    auto& crow = sm.p.crow;
+    auto& lrow = sm.p.lrow;
+    auto& raw = sm.p.raw;
+    auto& yb = sm.p.yb;
+    auto& dfac = sm.p.dfac;
+    auto& pcol = sm.p.pcol;
+    auto& gx = sm.p.gx;
+    for (int e = tid; e < 64; e += NT) cand[e >> 5][e & 31] = 0.0;
+    __syncthreads();
+    bool mine[R];   // row row0 + 64 r + lane not yet pivoted
+    int ppos[R];    // step of this panel that pivoted it, -1 if none
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int row = row0 + r * 64 + lane;
+        mine[r] = row < n && !((used[(row >> 5) & 31] >> (row & 31)) & 1u);
+        ppos[r] = -1;
+    }
+    int zero_col = 0;  // first zero pivot (1-based), uniform
+
+#pragma unroll 1
+    for (int g = 0; 4 * g < ncols; ++g) {
+        const int nc = min(4, ncols - 4 * g);
+        const int par = g & 1;
+        // the group's columns, one row per lane (a wave's own rows only; the
+        // empty asm keeps each copy a block of its own behind a uniform branch)
+#pragma unroll
+        for (int s = 0; s < NG; ++s)
+            if (s == g) {
+                asm volatile("");
+#pragma unroll
+                for (int i = 0; i < RB; ++i)
+                    gx[lk][row0 + i * 16 + li] = make_double2(accR[i][s / 4][s % 4], accI[i][s / 4][s % 4]);
+            }
+        double2 cur[R][4], am[R][4], dloc[4];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                cur[r][c] = gx[c][row0 + r * 64 + lane];
+                am[r][c] = make_double2(0.0, 0.0);
+            }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) dloc[c] = make_double2(0.0, 0.0);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (c >= nc) break;  // uniform
+            const int buf = c & 1;
+            // key: |re| + |im| with the low ten bits replaced by 1023 - row, so
+            // the maximum is the first row among equals (positive doubles order
+            // as their bits); 0 for rows already pivoted
+            double key = 0.0;
+            double2 best[4];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int row = row0 + r * 64 + lane;
+                const double a = cabs1(cur[r][c]);
+                double k = __hiloint2double(__double2hiint(a), (__double2loint(a) & ~1023) | (1023 - row));
+                k = mine[r] ? k : 0.0;
+                const bool up = r == 0 || k > key;
+                key = up ? k : key;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    best[e].x = up ? cur[r][e].x : best[e].x;
+                    best[e].y = up ? cur[r][e].y : best[e].y;
+                }
+            }
+            const double kmax = row16_max(key);
+            if (key == kmax) {
+                cand[buf][wave * 4 + lk] = key;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) crow[buf][wave * 4 + lk][e] = best[e];
+            }
+            __syncthreads();
+            const double top = row16_max(NW > 4 ? fmax(cand[buf][li], cand[buf][16 + li]) : cand[buf][li]);
+            const int tlo = __builtin_amdgcn_readfirstlane(__double2loint(top));
+            int p = 1023 - (tlo & 1023);
+            p = p < n ? p : 0;  // no finite candidate left
+            const int pw = p / (64 * R);  // its wave
+            const int slot = pw * 4 + ((p >> 4) & 3);
+            double2 u[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) u[e] = crow[buf][slot][e];
+            double2 d = crecip_fast(u[c]);
+            if (u[c].x == 0.0 && u[c].y == 0.0) {  // uniform
+                d = make_double2(0.0, 0.0);
+                zero_col = zero_col == 0 ? kb + 4 * g + c + 1 : zero_col;
+            }
+            dloc[c] = d;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const double2 gf = cmul(cur[r][c], d);  // f / pivot
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (e == c) continue;
+                    double2 t = cur[r][e];
+                    t.x = fma(-gf.x, u[e].x, t.x);
+                    t.x = fma(gf.y, u[e].y, t.x);
+                    t.y = fma(-gf.x, u[e].y, t.y);
+                    t.y = fma(-gf.y, u[e].x, t.y);
+                    cur[r][e] = t;
+                }
+                cur[r][c] = make_double2(-gf.x, -gf.y);
+                am[r][c] = gf;
+            }
+            if (pw == wave) {  // the pivot row itself stays, unscaled
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (row0 + r * 64 + lane == p) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) cur[r][e] = e == c ? make_double2(1.0, 0.0) : u[e];
+                        am[r][c] = make_double2(0.0, 0.0);
+                        mine[r] = false;
+                        ppos[r] = 4 * g + c;
+                        pcol[4 * g + c] = p;
+                        dfac[4 * g + c] = d;
+                    }
+            }
+        }
+        // multipliers for the update of the other columns (the pivot row of
+        // step c carries 1 / pivot_c there), and of the pivot rows for y
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int row = row0 + r * 64 + lane;
+            if (row < n) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const bool own = ppos[r] == 4 * g + c;
+                    double2 rec;
+                    rec.x = own ? dloc[c].x : am[r][c].x;
+                    rec.y = own ? dloc[c].y : am[r][c].y;
+                    if (c < nc) Gb[(unsigned)((4 * g + c) * n + row)] = rec;
+                }
+                if (ppos[r] >= 4 * g) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) lrow[par][ppos[r] - 4 * g][c] = am[r][c];
+                }
+            }
+        }
+        // back to the matrix layout: first the multipliers, then the columns
+        double2 gm[RB], gc[RB];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {  // (a pivot row takes the later steps only)
+                const bool before = c < ppos[r] - 4 * g;
+                gx[c][row0 + r * 64 + lane] =
+                    make_double2(before ? 0.0 : am[r][c].x, before ? 0.0 : am[r][c].y);
+            }
+#pragma unroll
+        for (int i = 0; i < RB; ++i) gm[i] = gx[lk][row0 + i * 16 + li];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) gx[c][row0 + r * 64 + lane] = cur[r][c];
+#pragma unroll
+        for (int i = 0; i < RB; ++i) gc[i] = gx[lk][row0 + i * 16 + li];
+        // the pivot rows as they were before the group, by the wave that holds them
+        bool any = false;
+#pragma unroll
+        for (int r = 0; r < R; ++r) any = any || ppos[r] >= 4 * g;
+        const bool hold = __ballot(any) != 0;
+        if (hold) {
+#pragma unroll
+            for (int i = 0; i < RB; ++i) {
+                const int pp = __shfl(ppos[i / 4], (i % 4) * 16 + li, 64) - 4 * g;
+                if (pp >= 0) {
+#pragma unroll
+                    for (int t = 0; t < NTL; ++t)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            raw[par][pp][16 * t + 4 * q + lk] = make_double2(accR[i][t][q], accI[i][t][q]);
+                }
+            }
+        }
+        __syncthreads();
+        // y of the group's steps at column 16 t + li, then the four steps on
+        // the panel's columns (the group's own are overwritten below)
+        const double2 l10 = lrow[par][1][0], l20 = lrow[par][2][0], l21 = lrow[par][2][1], l30 = lrow[par][3][0],
+                      l31 = lrow[par][3][1], l32 = lrow[par][3][2];
+        auto sub = [](double2 y, double2 l, double2 x) {
+            y.x = fma(-l.x, x.x, y.x);
+            y.x = fma(l.y, x.y, y.x);
+            y.y = fma(-l.x, x.y, y.y);
+            y.y = fma(-l.y, x.x, y.y);
+            return y;
+        };
+#pragma unroll
+        for (int t = 0; t < NTL; ++t) {
+            const double2 y0 = raw[par][0][16 * t + li];
+            const double2 y1 = sub(raw[par][1][16 * t + li], l10, y0);
+            const double2 y2 = sub(sub(raw[par][2][16 * t + li], l20, y0), l21, y1);
+            const double2 y3 = sub(sub(sub(raw[par][3][16 * t + li], l30, y0), l31, y1), l32, y2);
+            double2 bn;
+            bn.x = lk == 0 ? -y0.x : (lk == 1 ? -y1.x : (lk == 2 ? -y2.x : -y3.x));
+            bn.y = lk == 0 ? -y0.y : (lk == 1 ? -y1.y : (lk == 2 ? -y2.y : -y3.y));
+            bn.x = lk < nc ? bn.x : 0.0;
+            bn.y = lk < nc ? bn.y : 0.0;
+            const double bm = -bn.y;
+            if (hold) {  // a pivot row starts from the y the other rows see
+                yb[par][lk][16 * t + li] = make_double2(-bn.x, -bn.y);
+#pragma unroll
+                for (int i = 0; i < RB; ++i) {
+                    const int pp = __shfl(ppos[i / 4], (i % 4) * 16 + li, 64) - 4 * g;
+                    if (pp >= 0) {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const double2 y = yb[par][pp][16 * t + 4 * q + lk];
+                            accR[i][t][q] = y.x;
+                            accI[i][t][q] = y.y;
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < RB; ++i) {
+                accR[i][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(bn.x, gm[i].x, accR[i][t], 0, 0, 0);
+                accI[i][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(bn.y, gm[i].x, accI[i][t], 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < RB; ++i) {
+                accR[i][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(bm, gm[i].y, accR[i][t], 0, 0, 0);
+                accI[i][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(bn.x, gm[i].y, accI[i][t], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < NG; ++s)
+            if (s == g) {
+                asm volatile("");
+#pragma unroll
+                for (int i = 0; i < RB; ++i) {
+                    accR[i][s / 4][s % 4] = gc[i].x;
+                    accI[i][s / 4][s % 4] = gc[i].y;
+                }
+            }
+    }
+    __syncthreads();
+    if (tid < ncols) pv[kb + tid] = pcol[tid];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+        const int pp = __shfl(ppos[i / 4], (i % 4) * 16 + li, 64);
+        const int row = row0 + i * 16 + li;
+        if (row >= n) continue;
+        const double2 d = pp >= 0 ? dfac[pp] : make_double2(1.0, 0.0);
+#pragma unroll
+        for (int t = 0; t < NTL; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int col = 16 * t + 4 * q + lk;
+                const double2 v = make_double2(accR[i][t][q], accI[i][t][q]);
+                if (col < ncols) Ab[(unsigned)(row + (kb + col) * n)] = pp >= 0 ? cmul(v, d) : v;
+            }
+    }
+    if (tid == 0 && zero_col != 0 && info[b] == 0) info[b] = zero_col;
+}
+
 // ------------------------------------------------------------ output gather
 // X[r][c] = W[pivp[r]][pinv[c]]; zero block when the factorisation failed.
 __global__ __launch_bounds__(256) void gj_finish_kernel(const double2* W, int64_t sw, double2* X,
@@ -524,6 +1074,23 @@ void run_panels(hipStream_t s, const InvArgs& a) {
     }
 }
 
+// The multiplier records of two consecutive panels are alive at once (step k
+// reads panel k - 1's while it writes panel k's); they take turns in the first
+// 2 n kLaNB elements of the output block, which is written only at the end.
+template <int NW>
+void run_steps(hipStream_t s, const InvArgs& a) {
+    constexpr int NB = kLaNB;
+    const int n = a.n, ntiles = (n + NB - 1) / NB, npad = (a.batch + 7) / 8 * 8;
+    for (int k = 0; k <= ntiles; ++k) {
+        const int npan = k < ntiles ? npad : 0;
+        const int nupd = k > 0 ? npad * ntiles : 0;
+        hipLaunchKernelGGL((gj_step_kernel<NW>), dim3(npan + nupd), dim3(NW * 64), 0, s, a.A, a.sa,
+                           a.X + (size_t)((k + 1) & 1) * n * NB, a.X + (size_t)(k & 1) * n * NB, a.sx, n, a.batch, npan,
+                           ntiles, (k - 1) * NB, k < ntiles ? k * NB : -1, a.piv, a.info, a.active);
+        QT_HIP(hipGetLastError());
+    }
+}
+
 }  // namespace
 
 namespace {
@@ -537,7 +1104,15 @@ void zinv_part(hipStream_t s, const InvArgs& a) {
         return;
     }
     hipLaunchKernelGGL(zero_int_kernel, dim3((a.batch + 255) / 256), dim3(256), 0, s, a.info, a.batch);
-    if (n <= 256)
+    if (a.lookahead && n <= kLaMax) {
+        switch ((n + 63) / 64) {
+            case 2: run_steps<2>(s, a); break;
+            case 3: run_steps<3>(s, a); break;
+            case 4: run_steps<4>(s, a); break;
+            case 5: run_steps<5>(s, a); break;
+            default: run_steps<6>(s, a); break;
+        }
+    } else if (n <= 256)
         run_panels<32, 256>(s, a);
     else if (n <= 512)
         run_panels<32, 512>(s, a);
@@ -596,8 +1171,11 @@ int inv_parts() {
 
 }  // namespace
 
-// Blocks of n <= 64 take the one-launch kernel above on stream s.  For larger
-// ones, the panel kernel keeps one workgroup per member busy for a whole latency-
+// Blocks of n <= 64 take the one-launch kernel above on stream s, the look-ahead
+// steps overlap their own panels with the matrix work, and up to n = 256 the
+// panels of all members run at once (a split there costs: 100 members of 160
+// in the sweep's decimation, whole call 51.4 -> 47.5 ms without it).  For larger
+// blocks the panel kernel keeps one workgroup per member busy for a whole latency-
 // bound column sweep, leaving most CUs idle; the batch is therefore split in
 // parts on as many streams so that the panels of one part run while the
 // MFMA updates of the others fill the remaining CUs.
@@ -614,7 +1192,7 @@ void zinv(hipStream_t s, const InvArgs& a, Timer* t) {
     if (n > 1024) throw hip_error("zinv: block size above 1024", 6);
     if (!a.G || a.sg < (int64_t)n * kInvPanelMax) throw hip_error("zinv: multiplier workspace missing", 1);
     if (t && t->enabled) t->begin(s, 1);
-    if (a.batch >= 8 && n > 64) {
+    if (a.batch >= 8 && n > 256 && !(a.lookahead && n <= kLaMax)) {
         Side& sd = side();
         const int parts = std::min(inv_parts(), a.batch / 4);
         QT_HIP(hipEventRecord(sd.fork, s));

@@ -710,7 +710,7 @@ int qt_lead_surface(qt_lead* l, int32_t mode, int32_t flags, int32_t npts, const
                     sh.c1 = -1.0;
                     sh.kidx = lw.kidx;
                     shifted(s, sh);
-                    inv_batch(c, w, n, M, w.T[0], nn, lw.g, nn, nullptr);
+                    inv_batch(c, w, n, M, w.T[0], nn, lw.g, nn, nullptr, -1, false);
                 }
                 copy_blocks(s, n, M, lw.g0, nn, op_member(lw.g, n, nn), nullptr, 0, false);
                 rep.network_ms += cn.stop(s);
@@ -745,7 +745,7 @@ int qt_lead_surface(qt_lead* l, int32_t mode, int32_t flags, int32_t npts, const
                     sh.kidx = lw.kidx;
                     sh.active = lw.act;
                     shifted(s, sh);
-                    inv_batch(c, w, n, M, Ashift, nn, Mi, nn, lw.act, nact);
+                    inv_batch(c, w, n, M, Ashift, nn, Mi, nn, lw.act, nact, false);
                     combine(s, nn, M, r, 1.0, Mi, -1.0, lw.g, lw.act);  // r = Phi(g) - g
                     norm2(s, M, r, nullptr, nn, lw.act, lw.n1);
                     norm2(s, M, Mi, nullptr, nn, lw.act, lw.n2);

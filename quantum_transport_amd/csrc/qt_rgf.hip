@@ -112,7 +112,7 @@ void work_carve(Arena& a, Work& w, const qt_ham& h, int B, bool sigma, bool keep
 }
 
 void inv_batch(Ctx& c, Work& w, int n, int batch, double2* A, int64_t sa, double2* X,
-               int64_t sx, const int* active, int flop_batch) {
+               int64_t sx, const int* active, int flop_batch, bool lookahead) {
     InvArgs a;
     a.n = n;
     a.batch = batch;
@@ -126,6 +126,7 @@ void inv_batch(Ctx& c, Work& w, int n, int batch, double2* A, int64_t sa, double
     a.sg = (int64_t)n * kInvPanelMax;
     a.active = active;
     a.flop_batch = flop_batch;
+    a.lookahead = lookahead;
     zinv(c.stream, a, &c.timer);
 }
 
@@ -159,6 +160,7 @@ void sancho_run(Ctx& c, Work& w, SanchoIO& io) {
     copy_blocks(s, n, M, HBB, nn, io.H00, io.kidx, 0, false);
     copy_blocks(s, n, M, H01, nn, op_member(H10, n, nn), nullptr, 0, true);
     const bool dual = io.G00b != nullptr;
+    const bool la = io.eta >= kLookaheadEta;
     double2* HSS2 = T[14];
     if (dual) {
         copy_blocks(s, n, M, HSS2, nn, io.H00, io.kidx, 0, false);
@@ -188,7 +190,7 @@ void sancho_run(Ctx& c, Work& w, SanchoIO& io) {
         sh.kidx = io.kidx;
         sh.active = w.active;
         shifted(s, sh);                                   // A = z S00 - H_BB
-        inv_batch(c, w, n, M, A, nn, Ai, nn, w.active, nact);  // invert(A)
+        inv_batch(c, w, n, M, A, nn, Ai, nn, w.active, nact, la);  // invert(A)
         const ZOp a = op_member(Ai, n, nn), h10 = op_member(H10, n, nn), h01 = op_member(H01, n, nn);
         g(OP_N, OP_N, n, n, n, a, h10, B1, n, nn);                       // B = A H_10
         g(OP_N, OP_N, n, n, n, h01, op_member(B1, n, nn), C1, n, nn);    // C = H_01 B
@@ -253,7 +255,7 @@ void sancho_run(Ctx& c, Work& w, SanchoIO& io) {
         sh.c1 = -1.0;
         sh.kidx = io.kidx;
         shifted(s, sh);
-        inv_batch(c, w, n, M, A, nn, io.G00b, nn, nullptr);
+        inv_batch(c, w, n, M, A, nn, io.G00b, nn, nullptr, -1, la);
         if (io.info_bits) note_inv_info(c, w, M, io.period);
     }
     for (int pass = 0; pass < (io.GBB ? 2 : 1); ++pass) {
@@ -269,7 +271,7 @@ void sancho_run(Ctx& c, Work& w, SanchoIO& io) {
         sh.c1 = -1.0;
         sh.kidx = io.kidx;
         shifted(s, sh);
-        inv_batch(c, w, n, M, A, nn, pass == 0 ? io.G00 : io.GBB, nn, nullptr);
+        inv_batch(c, w, n, M, A, nn, pass == 0 ? io.G00 : io.GBB, nn, nullptr, -1, la);
         if (io.info_bits) note_inv_info(c, w, M, io.period);
     }
 }
@@ -1586,6 +1588,7 @@ int qt_invert_batched_noalloc(int32_t n, int32_t batch, void* A, void* X, int32_
         a.info = sinfo;  // cleared by the inversion itself
         a.G = G;
         a.sg = (int64_t)n * kInvPanelMax;
+        a.lookahead = true;
         zinv_single(c.stream, a);
         hipLaunchKernelGGL(info_any_kernel, dim3((batch + 255) / 256), dim3(256), 0, c.stream, sinfo, batch,
                            flag);
