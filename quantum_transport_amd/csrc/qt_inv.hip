@@ -73,13 +73,24 @@ __device__ __forceinline__ double dpp_max_step(double x) {
     const int thi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWMASK, 0xF, false);
     return fmax(x, __hiloint2double(thi, tlo));
 }
-// maximum over the 64 lanes (row shifts 1, 2, 4, 8 leave each 16-lane
-// row's maximum in its last lane; row broadcasts 15 and 31 carry it to lane 63)
+template <int CTRL>
+__device__ __forceinline__ double dpp_rotate(double x) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), CTRL, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+// maximum over each 16-lane row, in every lane (rotations by 8, 4, 2, 1)
+__device__ __forceinline__ double row16_max(double x) {
+    x = fmax(x, dpp_rotate<0x128>(x));
+    x = fmax(x, dpp_rotate<0x124>(x));
+    x = fmax(x, dpp_rotate<0x122>(x));
+    return fmax(x, dpp_rotate<0x121>(x));
+}
+
+// maximum over the 64 lanes: every 16-lane row's by rotations, then row
+// broadcasts 15 and 31 carry it to lane 63
 __device__ __forceinline__ double wave_max(double x) {
-    x = dpp_max_step<0x111, 0xF>(x);
-    x = dpp_max_step<0x112, 0xF>(x);
-    x = dpp_max_step<0x114, 0xF>(x);
-    x = dpp_max_step<0x118, 0xF>(x);
+    x = row16_max(x);
     x = dpp_max_step<0x142, 0xA>(x);
     x = dpp_max_step<0x143, 0xC>(x);
     const int lo = __builtin_amdgcn_readlane(__double2loint(x), 63);
@@ -363,20 +374,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void gj
 // ------------------------------------------------------------ look-ahead steps
 constexpr int kLaNB = 32;   // panel and tile width
 constexpr int kLaMax = 384;  // largest block: six waves of 64 rows
-
-template <int CTRL>
-__device__ __forceinline__ double dpp_rotate(double x) {
-    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), CTRL, 0xF, 0xF, true);
-    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), CTRL, 0xF, 0xF, true);
-    return __hiloint2double(hi, lo);
-}
-// maximum over each 16-lane row, in every lane (rotations by 8, 4, 2, 1)
-__device__ __forceinline__ double row16_max(double x) {
-    x = fmax(x, dpp_rotate<0x128>(x));
-    x = fmax(x, dpp_rotate<0x124>(x));
-    x = fmax(x, dpp_rotate<0x122>(x));
-    return fmax(x, dpp_rotate<0x121>(x));
-}
 
 // 1 / (a.x + i a.y) with one reciprocal, refined by two Newton steps (the
 // hardware seed has more than 20 correct bits), of |a|^2; operands whose
@@ -936,8 +933,8 @@ __global__ __launch_bounds__(256) void gj_finish_kernel(const double2* W, int64_
 }
 
 // ------------------------------------------------------------ blocks of n <= 64
-// The whole inversion in one launch: one 256-thread workgroup per member,
-// wave w holding columns 16 w .. 16 w + 15, lane r holding row r, in
+// The whole inversion in one launch: one workgroup of 8 waves (4 up to n = 32)
+// per member, wave w holding columns 8 w .. 8 w + 7, lane r holding row r, in
 // registers.  Unblocked Gauss-Jordan with the pivot rule and the row
 // operations of the panel kernel (first-indexed maximal |re| + |im| among the
 // rows not yet pivoted, the pivot row kept unscaled with its factor 1/pivot
@@ -956,7 +953,14 @@ __device__ __forceinline__ double readlane_f64(double x, int l) {
     return __hiloint2double(hi, lo);
 }
 
-__global__ __launch_bounds__(256) void gj_small_kernel(const double2* A, int64_t sa, double2* X, int64_t sx,
+//
+// Bound by the column's chain (search, barrier, reciprocal, readlanes).  Eight
+// columns a wave instead of sixteen leave 32 x 32 blocks half the readlanes: one
+// block, call included, 52 -> 43 us; FAST (InvArgs::lookahead) takes one
+// refined reciprocal instead of Smith's three dependent divisions: 41 us, and
+// 256 of 64 x 64 88 -> 81 us.
+template <int NWS, bool FAST>
+__global__ __launch_bounds__(NWS * 64) void gj_small_kernel(const double2* A, int64_t sa, double2* X, int64_t sx,
                                                        int n, int* info, const int* active) {
     const int b = blockIdx.x;
     if (active && !active[b]) {
@@ -971,20 +975,20 @@ __global__ __launch_bounds__(256) void gj_small_kernel(const double2* A, int64_t
     __shared__ int zero_s;
     const int t = threadIdx.x, r = t & 63, w = t >> 6;
     const double2* Ab = A + b * sa;
-    double2 v[16];
+    double2 v[8];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const int c = 16 * w + k;
+    for (int k = 0; k < 8; ++k) {
+        const int c = 8 * w + k;
         v[k] = (r < n && c < n) ? Ab[r + c * n] : make_double2(0.0, 0.0);
     }
     bool mine = r < n;  // row not yet pivoted
     double2 srow = make_double2(1.0, 0.0);
     int zero_col = 0;   // first zero pivot (1-based), thread 0
 #pragma unroll 1
-    for (int jw = 0; jw < 4; ++jw) {
+    for (int jw = 0; jw < NWS; ++jw) {
 #pragma unroll
-        for (int jj = 0; jj < 16; ++jj) {
-            const int j = 16 * jw + jj;
+        for (int jj = 0; jj < 8; ++jj) {
+            const int j = 8 * jw + jj;
             if (j >= n) continue;  // uniform over the workgroup
             const int buf = j & 1;
             if (w == jw) {  // the wave holding column j
@@ -1002,7 +1006,8 @@ __global__ __launch_bounds__(256) void gj_small_kernel(const double2* A, int64_t
             if (p < 0 || p >= n) p = 0;  // unreachable: n - j rows are always unpivoted
             const double2 f = fcol[buf][r];
             const double2 pivv = fcol[buf][p];
-            const double2 d = (pivv.x == 0.0 && pivv.y == 0.0) ? make_double2(0.0, 0.0) : crecip(pivv);
+            const double2 d = (pivv.x == 0.0 && pivv.y == 0.0) ? make_double2(0.0, 0.0)
+                                                                  : (FAST ? crecip_fast(pivv) : crecip(pivv));
             if (t == 0) {
                 pvs[j] = p;
                 pinv[p] = j;
@@ -1013,7 +1018,7 @@ __global__ __launch_bounds__(256) void gj_small_kernel(const double2* A, int64_t
             // every row but the pivot row: v -= gf * (pivot row); the pivot
             // row's value of column k is read from lane p before it changes
 #pragma unroll
-            for (int k = 0; k < 16; ++k) {
+            for (int k = 0; k < 8; ++k) {
                 const double ux = readlane_f64(v[k].x, p), uy = readlane_f64(v[k].y, p);
                 double2 x = v[k];
                 x.x = fma(-gf.x, ux, x.x);
@@ -1043,8 +1048,8 @@ __global__ __launch_bounds__(256) void gj_small_kernel(const double2* A, int64_t
     double2* Xb = X + b * sx;
     const int orow = pinv[r];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        const int c = 16 * w + k;
+    for (int k = 0; k < 8; ++k) {
+        const int c = 8 * w + k;
         if (c >= n) continue;
         const double2 o = bad ? make_double2(0.0, 0.0) : cmul(v[k], srow);
         Xb[orow + (int64_t)pvs[c] * n] = o;
@@ -1098,8 +1103,13 @@ namespace {
 void zinv_part(hipStream_t s, const InvArgs& a) {
     const int n = a.n;
     if (n <= 64) {
-        hipLaunchKernelGGL(gj_small_kernel, dim3(a.batch), dim3(256), 0, s, a.A, a.sa, a.X, a.sx, n, a.info,
-                           a.active);
+        auto launch = [&](auto kernel, int waves) {
+            hipLaunchKernelGGL(kernel, dim3(a.batch), dim3(64 * waves), 0, s, a.A, a.sa, a.X, a.sx, n, a.info, a.active);
+        };
+        if (n <= 32)
+            a.lookahead ? launch(gj_small_kernel<4, true>, 4) : launch(gj_small_kernel<4, false>, 4);
+        else
+            a.lookahead ? launch(gj_small_kernel<8, true>, 8) : launch(gj_small_kernel<8, false>, 8);
         QT_HIP(hipGetLastError());
         return;
     }
