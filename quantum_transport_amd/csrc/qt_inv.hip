@@ -947,18 +947,18 @@ __global__ __launch_bounds__(256) void gj_finish_kernel(const double2* W, int64_
 // by its factor) and the zero block of a failed factorisation are written by
 // the same workgroup.  A and X may be the same array: every element of A is
 // read before the first barrier and X is written after the last one.
-__device__ __forceinline__ double readlane_f64(double x, int l) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(x), l);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(x), l);
-    return __hiloint2double(hi, lo);
-}
-
 //
 // Bound by the column's chain (search, barrier, reciprocal, readlanes).  Eight
 // columns a wave instead of sixteen leave 32 x 32 blocks half the readlanes: one
 // block, call included, 52 -> 43 us; FAST (InvArgs::lookahead) takes one
 // refined reciprocal instead of Smith's three dependent divisions: 41 us, and
 // 256 of 64 x 64 88 -> 81 us.
+__device__ __forceinline__ double readlane_f64(double x, int l) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(x), l);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(x), l);
+    return __hiloint2double(hi, lo);
+}
+
 template <int NWS, bool FAST>
 __global__ __launch_bounds__(NWS * 64) void gj_small_kernel(const double2* A, int64_t sa, double2* X, int64_t sx,
                                                        int n, int* info, const int* active) {
