@@ -697,16 +697,19 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
             if (c >= nc) break;  // uniform
             const int buf = c & 1;
             // key: |re| + |im| with the low ten bits replaced by 1023 - row, so
-            // the maximum is the first row among equals (positive doubles order
-            // as their bits); 0 for rows already pivoted
+            // the maximum is the first row among those equal to it in the other
+            // bits (positive doubles order as their bits).  An infinite entry
+            // counts as the largest finite one; 0 for rows already pivoted and
+            // for a NaN, so that every key is a number
             double key = 0.0;
             double2 best[4];
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const int row = row0 + r * 64 + lane;
                 const double a = cabs1(cur[r][c]);
-                double k = __hiloint2double(__double2hiint(a), (__double2loint(a) & ~1023) | (1023 - row));
-                k = mine[r] ? k : 0.0;
+                const int hi = __double2hiint(a), lo = hi > 0x7fefffff ? ~0 : __double2loint(a);
+                double k = __hiloint2double(min(hi, 0x7fefffff), (lo & ~1023) | (1023 - row));
+                k = mine[r] && a == a ? k : 0.0;
                 const bool up = r == 0 || k > key;
                 key = up ? k : key;
 #pragma unroll
@@ -725,14 +728,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
             const double top = row16_max(NW > 4 ? fmax(cand[buf][li], cand[buf][16 + li]) : cand[buf][li]);
             const int tlo = __builtin_amdgcn_readfirstlane(__double2loint(top));
             int p = 1023 - (tlo & 1023);
-            p = p < n ? p : 0;  // no finite candidate left
+            const bool none = p >= n;  // top = 0: every row left is a NaN
+            p = none ? 0 : p;
             const int pw = p / (64 * R);  // its wave
             const int slot = pw * 4 + ((p >> 4) & 3);
             double2 u[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) u[e] = crow[buf][slot][e];
             double2 d = crecip_fast(u[c]);
-            if (u[c].x == 0.0 && u[c].y == 0.0) {  // uniform
+            if (none || (u[c].x == 0.0 && u[c].y == 0.0)) {  // uniform
                 d = make_double2(0.0, 0.0);
                 zero_col = zero_col == 0 ? kb + 4 * g + c + 1 : zero_col;
             }
@@ -913,6 +917,13 @@ __global__ __launch_bounds__(256) void gj_finish_kernel(const double2* W, int64_
     if (active && !active[b]) return;
     __shared__ int rows[1024];
     __shared__ int pinv[1024];
+    double2* Xb = X + b * sx;
+    const int c0 = blockIdx.x * 8, c1 = min(c0 + 8, n);
+    if (info[b] != 0) {  // its list may name a row twice, so that pinv would have gaps
+        for (int c = c0; c < c1; ++c)
+            for (int r = threadIdx.x; r < n; r += 256) Xb[r + (int64_t)c * n] = make_double2(0.0, 0.0);
+        return;
+    }
     const int* pv = pivp + (int64_t)b * n;
     for (int i = threadIdx.x; i < n; i += 256) {
         const int p = pv[i];
@@ -920,15 +931,11 @@ __global__ __launch_bounds__(256) void gj_finish_kernel(const double2* W, int64_
         pinv[p] = i;
     }
     __syncthreads();
-    const bool bad = info[b] != 0;
     const double2* Wb = W + b * sw;
-    double2* Xb = X + b * sx;
-    for (int cc = 0; cc < 8; ++cc) {
-        const int c = blockIdx.x * 8 + cc;
-        if (c >= n) break;
+    for (int c = c0; c < c1; ++c) {
         const double2* src = Wb + (int64_t)pinv[c] * n;
         double2* dst = Xb + (int64_t)c * n;
-        for (int r = threadIdx.x; r < n; r += 256) dst[r] = bad ? make_double2(0.0, 0.0) : src[rows[r]];
+        for (int r = threadIdx.x; r < n; r += 256) dst[r] = src[rows[r]];
     }
 }
 

@@ -1,0 +1,83 @@
+"""Blocks with a NaN among their entries beside regular ones: the pivot search takes no NaN while a number is
+left, so the elimination ends at the first column whose remaining rows are all NaN (or zero); info names that
+column, the block is zeroed and the other members are untouched."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [65, 96, 97, 128, 160, 255, 257, 384, 385]
+
+
+@pytest.fixture(scope="module")
+def qt():
+    from quantum_transport_amd import rgf
+
+    rgf.init(0)
+    return rgf
+
+
+def _info(A):
+    """First column (1-based) without a pivot in unblocked Gauss-Jordan by components: the largest |re| + |im|
+    among the rows not yet taken, a NaN never; 0 if every column has one."""
+    n = len(A)
+    re, im = A.real.copy(), A.imag.copy()
+    left = np.ones(n, bool)
+    with np.errstate(all="ignore"):
+        for j in range(n):
+            key = np.where(left, np.abs(re[:, j]) + np.abs(im[:, j]), -1.0)
+            if not np.fmax.reduce(key) > 0.0:
+                return j + 1
+            p = int(np.nanargmax(key))
+            left[p] = False
+            x, y = re[p, j], im[p, j]
+            if abs(x) >= abs(y):
+                r = y / x
+                d = x + y * r
+                dx, dy = 1.0 / d, -r / d
+            else:
+                r = x / y
+                d = y + x * r
+                dx, dy = r / d, -1.0 / d
+            gx, gy = re[:, j] * dx - im[:, j] * dy, re[:, j] * dy + im[:, j] * dx
+            ur, ui = re[p].copy(), im[p].copy()
+            re -= np.outer(gx, ur) - np.outer(gy, ui)
+            im -= np.outer(gx, ui) + np.outer(gy, ur)
+            re[:, j], im[:, j] = -gx, -gy
+            re[p], im[p], re[p, j], im[p, j] = ur, ui, 1.0, 0.0
+    return 0
+
+
+def _blocks(n):
+    rng = np.random.default_rng(n)
+    blk = lambda: rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n)) + 4.0 * np.sqrt(n) * np.eye(n)
+    bad = {}
+    for name, r, c in (("first", 0, 0), ("last", n - 1, n - 1), ("inside", n // 2, n // 3), ("corner", n - 1, 0)):
+        bad[name] = blk()
+        bad[name][r, c] = np.nan
+    for name, at in (("row", np.s_[n // 2]), ("column", np.s_[:, n // 2]), ("lanes 16-31", np.s_[16:32]),
+                     ("all", np.s_[:]), ("imaginary part", np.s_[n // 3, 1])):
+        bad[name] = blk()
+        bad[name][at] = complex(1.0, np.nan) if name == "imaginary part" else np.nan
+    bad["tiny pivots"] = blk() * 1e-312  # their reciprocals overflow
+    return blk, bad
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_blocks_with_nan(qt, n):
+    blk, bad = _blocks(n)
+    A = []
+    for B in bad.values():
+        A += [blk(), B]
+    A = np.stack(A + [blk()])
+    regular = A.copy()
+    regular[1::2] = [blk() for _ in bad]
+    print("n", n, "blocks with NaN", len(bad), flush=True)
+    X, info = qt.invert_batched(A)
+    ref, ref_info = qt.invert_batched(regular)
+    assert not ref_info.any()
+    assert np.array_equal(X[0::2], ref[0::2]) and not info[0::2].any()
+    for i, (name, B) in enumerate(bad.items()):
+        want = _info(B)
+        assert want > 0 and info[2 * i + 1] == want, name
+        assert not X[2 * i + 1].any(), name
