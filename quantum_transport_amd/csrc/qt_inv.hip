@@ -174,7 +174,7 @@ __global__ __launch_bounds__(NT) void gj_panel_loop_kernel(double2* A, int64_t s
         const unsigned long long hitw = __ballot(rvv == bv);
         int p = __builtin_amdgcn_readlane(riv, __ffsll((long long)hitw) - 1);
         const int j = kb + c;
-        if (p < 0 || p >= n) p = 0;  // unreachable: n - j rows are always unpivoted
+        if (p < 0 || p >= n) p = 0;  // every row left is a NaN (bv is then not positive)
         if (r == p) {
 #pragma unroll
             for (int cc = 0; cc < NB; ++cc) prow[buf][cc] = v[cc];
@@ -1010,7 +1010,7 @@ __global__ __launch_bounds__(NWS * 64) void gj_small_kernel(const double2* A, in
             }
             __syncthreads();
             int p = __builtin_amdgcn_readfirstlane(piv_s[buf]);
-            if (p < 0 || p >= n) p = 0;  // unreachable: n - j rows are always unpivoted
+            if (p < 0 || p >= n) p = 0;  // every row left is a NaN (the maximum is then not positive)
             const double2 f = fcol[buf][r];
             const double2 pivv = fcol[buf][p];
             const double2 d = (pivv.x == 0.0 && pivv.y == 0.0) ? make_double2(0.0, 0.0)
@@ -1053,13 +1053,13 @@ __global__ __launch_bounds__(NWS * 64) void gj_small_kernel(const double2* A, in
     const bool bad = zero_s != 0;
     if (r >= n) return;
     double2* Xb = X + b * sx;
-    const int orow = pinv[r];
+    const int orow = bad ? r : pinv[r];  // a failed block's list may name a row twice: pinv has gaps
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
         const int c = 8 * w + k;
         if (c >= n) continue;
         const double2 o = bad ? make_double2(0.0, 0.0) : cmul(v[k], srow);
-        Xb[orow + (int64_t)pvs[c] * n] = o;
+        Xb[orow + (bad ? c : pvs[c]) * n] = o;
     }
 }
 

@@ -6,7 +6,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [65, 96, 97, 128, 160, 255, 257, 384, 385]
+SIZES = [1, 2, 31, 32, 33, 63, 64, 65, 96, 97, 128, 160, 255, 257, 384, 385]
 
 
 @pytest.fixture(scope="module")
@@ -56,10 +56,15 @@ def _blocks(n):
         bad[name] = blk()
         bad[name][r, c] = np.nan
     for name, at in (("row", np.s_[n // 2]), ("column", np.s_[:, n // 2]), ("lanes 16-31", np.s_[16:32]),
-                     ("all", np.s_[:]), ("imaginary part", np.s_[n // 3, 1])):
+                     ("all", np.s_[:])):
         bad[name] = blk()
-        bad[name][at] = complex(1.0, np.nan) if name == "imaginary part" else np.nan
-    bad["tiny pivots"] = blk() * 1e-312  # their reciprocals overflow
+        bad[name][at] = np.nan
+    bad["imaginary part"] = blk()
+    bad["imaginary part"][n // 3, n // 2] = complex(1.0, np.nan)
+    if n <= 16:
+        del bad["lanes 16-31"]
+    if n > 1:
+        bad["tiny pivots"] = blk() * 1e-312  # their reciprocals overflow
     return blk, bad
 
 
