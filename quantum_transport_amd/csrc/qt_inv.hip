@@ -37,6 +37,7 @@
 // A zero pivot sets info (first column, 1-based) and the output block is
 // zeroed (linalg.f90:50-58).
 #include <algorithm>
+#include <cfloat>
 #include <climits>
 #include <cstdlib>
 
@@ -378,15 +379,18 @@ constexpr int kLaMax = 384;  // largest block: six waves of 64 rows
 // 1 / (a.x + i a.y) with one reciprocal, refined by two Newton steps (the
 // hardware seed has more than 20 correct bits), of |a|^2; operands whose
 // squares would leave the normal range are scaled by a power of two first.
-// (Smith's form takes three dependent divisions.)  a is uniform over the wave.
+// (Smith's form takes three dependent divisions.)  As there, one infinite part
+// makes the reciprocal zero, two make it NaN.  a is uniform over the wave.
 __device__ __forceinline__ double2 crecip_fast(double2 a) {
     double t = fma(a.x, a.x, a.y * a.y);
     int e = 0;
     if (!(t > 1e-280 && t < 1e280)) {
-        e = __builtin_amdgcn_frexp_exp(fmax(fabs(a.x), fabs(a.y)));
-        a.x = ldexp(a.x, -e);
-        a.y = ldexp(a.y, -e);
-        t = fma(a.x, a.x, a.y * a.y);
+        const double m = fmax(fabs(a.x), fabs(a.y)), q = 0.0 * fmin(fabs(a.x), fabs(a.y));
+        const bool inf = m > DBL_MAX;
+        e = __builtin_amdgcn_frexp_exp(m);  // 0 for an infinity
+        a.x = inf ? q : ldexp(a.x, -e);
+        a.y = inf ? q : ldexp(a.y, -e);
+        t = inf ? 1.0 : fma(a.x, a.x, a.y * a.y);
     }
     double r = __builtin_amdgcn_rcp(t);
     r = fma(r, fma(-t, r, 1.0), r);

@@ -1,6 +1,7 @@
 """Blocks with a NaN among their entries beside regular ones: the pivot search takes no NaN while a number is
 left, so the elimination ends at the first column whose remaining rows are all NaN (or zero); info names that
-column, the block is zeroed and the other members are untouched."""
+column, the block is zeroed and the other members are untouched.  An infinite pivot is an ordinary one with
+reciprocal zero: its row and column of the inverse are zero and the rest is the inverse without them."""
 import numpy as np
 import pytest
 
@@ -86,3 +87,25 @@ def test_blocks_with_nan(qt, n):
         want = _info(B)
         assert want > 0 and info[2 * i + 1] == want, name
         assert not X[2 * i + 1].any(), name
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_infinite_pivot(qt, n):
+    rng = np.random.default_rng(n)
+    blk = lambda: (rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))
+                   + (8.0 + 4.0 * np.sqrt(n)) * np.eye(n))  # every column's pivot is its diagonal entry
+    where = [(r, v) for r in sorted({0, n // 2, n - 1})
+             for v in (complex(np.inf, 1.0), complex(-1.0, -np.inf), complex(-np.inf, 0.0))]
+    A = np.stack([blk() for _ in where] + [blk()])
+    for b, (r, v) in enumerate(where):
+        A[b, r, r] = v
+    print("n", n, "blocks with an infinite pivot", len(where), flush=True)
+    X, info = qt.invert_batched(A)
+    assert not info.any()
+    assert np.array_equal(X[-1], qt.invert_batched(A[-1:])[0][0])
+    for b, (r, v) in enumerate(where):
+        assert not X[b, r].any() and not X[b, :, r].any(), (r, v)
+        rest = np.delete(np.arange(n), r)
+        a, x = A[b][np.ix_(rest, rest)], X[b][np.ix_(rest, rest)]
+        bound = 8 * n * np.finfo(float).eps * np.linalg.norm(a) * np.linalg.norm(x)
+        assert n == 1 or np.abs(a @ x - np.eye(n - 1)).max() <= bound, (r, v)
