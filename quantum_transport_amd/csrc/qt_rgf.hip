@@ -23,6 +23,7 @@
 
 #include "../../include/qt_rgf.h"
 #include "qt_ctx.h"
+#include "qt_plan.h"
 #include "qt_internal.h"
 
 
@@ -1070,33 +1071,17 @@ int qt_ham_destroy(qt_ham* h) {
     return QT_OK;
 }
 
-// Whether the first pass's coupling products stay resident: where 32 points
-// with them fit the device's memory.  It depends on the device and the shape
-// only, so a point's results do not depend on what else is allocated.
-static bool keep_products(const qt_ham& h, bool sigma) {
+// QT_BATCH sets the points of a batch, QT_WORKSET_BYTES bounds what kept products
+// and more than 128 points take
+static BatchPlan plan_points(const qt_ham& h, int npts, bool sigma) {
+    const char *batch = getenv("QT_BATCH"), *workset = getenv("QT_WORKSET_BYTES");
     size_t freeb = 0, total = 0;
-    if (hipMemGetInfo(&freeb, &total) != hipSuccess) return false;
-    return work_bytes(h, 32, sigma, true) <= (size_t)(0.80 * (double)total);
-}
-
-// Points per device batch.  A product of n x n blocks is ceil(n / 64)^2
-// workgroups a member and the device takes 512 at once, so small blocks need
-// more members than the 128 that fill it from n = 192 on (n = 64, 256 points:
-// 256 members take the sweep of 32 slabs from 23.8 to
-// 12.9 ms).  The points are dealt evenly: a batch is
-// padded to B by repeating a point.
-static int choose_batch(qt_ham& h, int npts, bool sigma, bool keep) {
-    const char* env = getenv("QT_BATCH");
-    if (env && atoi(env) > 0) return std::min(npts, atoi(env));
-    size_t freeb = 0, total = 0;
-    if (hipMemGetInfo(&freeb, &total) != hipSuccess) freeb = (size_t)8 << 30;
-    const size_t budget = (size_t)(0.80 * (double)(freeb + g_ctx->arena.cap));
-    const int tiles = ((h.nmax + 63) / 64) * ((h.nmax + 63) / 64);
-    int B = std::min(npts, std::max(128, 1024 / tiles));
-    while (B > 1 && work_bytes(h, B, sigma, keep) > budget) B = B * 3 / 4;
-    B = std::max(B, 1);
-    const int parts = (npts + B - 1) / B;
-    return (npts + parts - 1) / parts;
+    if (hipMemGetInfo(&freeb, &total) != hipSuccess) {
+        freeb = (size_t)8 << 30;
+        total = 0;
+    }
+    return plan_batch(npts, h.nmax, freeb + g_ctx->arena.cap, total, workset ? (size_t)std::max(atoll(workset), 0ll) : 0,
+                      batch ? atoi(batch) : 0, [&](int B, bool keep) { return work_bytes(h, B, sigma, keep); });
 }
 
 int qt_rgf_solve(qt_ham* h, const qt_rgf_params* p, int32_t npts, const double* En,
@@ -1121,8 +1106,7 @@ int qt_rgf_solve(qt_ham* h, const qt_rgf_params* p, int32_t npts, const double* 
     std::lock_guard<std::mutex> lk(c.mu);
     try {
         QT_HIP(hipSetDevice(c.device));
-        const bool keep = keep_products(*h, sigma);
-        const int B = choose_batch(*h, npts, sigma, keep);
+        const auto [B, keep] = plan_points(*h, npts, sigma);
         c.arena.reserve(work_bytes(*h, B, sigma, keep));
         Work w;
         work_carve(c.arena, w, *h, B, sigma, keep);
@@ -2483,8 +2467,7 @@ int qt_gw_scba_step(qt_ham* h, const qt_rgf_params* p, int32_t nen, const double
 
         // ---- G of every energy (qt_rgf_solve's batch loop, QT_RGF_GW with sigma)
         {
-            const bool keep = keep_products(*h, true);
-            const int B = choose_batch(*h, nen, true, keep);
+            const auto [B, keep] = plan_points(*h, nen, true);
             c.arena.reserve(work_bytes(*h, B, true, keep));
             Work w;
             work_carve(c.arena, w, *h, B, true, keep);

@@ -2,7 +2,8 @@
 devices whose neighbouring slabs take the Z form (equal sizes) and the other
 one in turn, couplings that differ from slab to slab (the first pass's products
 are then not those of the reference's forward second pass), and diagonals that
-do not depend on whether the blocks are asked for too.  The contacts are
+do not depend on whether the blocks are asked for too, and the sweep without the
+first pass's products (memory refused).  The contacts are
 broadened by 10 meV; every point is held to the parity bar of the sweep tests,
 relative to the largest block of the recursion."""
 import numpy as np
@@ -108,3 +109,17 @@ def test_diagonals_with_and_without_blocks(qt, n, slabs, variant):
             G, gl = b["G_r"][p][s], b["Gl"][p][s]
             tol = 8 * n * n * np.finfo(float).eps * (np.abs(G).max() + np.abs(gl).max())
             assert np.abs(np.diagonal(G) - a["gr_diag"][p, s * n:(s + 1) * n]).max() <= tol
+
+
+@pytest.mark.parametrize("sizes,variant", [([33] * 5, "forward"), ([65] * 4, "backward"), ([20, 20, 64, 64, 33], "forward")])
+def test_products_not_kept(qt, oracle_mod, monkeypatch, sizes, variant):
+    monkeypatch.setenv("QT_WORKSET_BYTES", "1")
+    uneven = len(set(sizes)) > 1
+    dev = (hm.uneven_device(sizes, seed=23, coupling_density=0.2) if uneven
+           else hm.synthetic_device(sizes[0], len(sizes), seed=31, coupling_density=0.2)[1])
+    _check(qt, oracle_mod, dev, variant, fix=uneven)
+    # and blocks of up to 64 go back to 128 points a batch
+    H = qt.Hamiltonian.from_device(dev)
+    qt.solve_batch(H, hm.energy_grid(-0.25, 0.15, 140), None, variant=variant, coupling_fix=uneven, lead_eta=ETA)
+    H.close()
+    assert qt.last_timing()["batch"] == 70
