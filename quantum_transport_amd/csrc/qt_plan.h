@@ -21,7 +21,9 @@ struct BatchPlan {
 // More points: a product of n x n blocks is ceil(n / 64)^2 workgroups a member and
 // the device takes 512 at once, so blocks of up to 128 need more members to fill
 // it: up to 1024 workgroups (n = 64, 256 points: 256 members take the sweep of
-// 32 slabs from 23.8 to 12.9 ms).
+// 32 slabs from 23.8 to 12.9 ms).  The workspace is held until the library is
+// finished, so they stop at a sixteenth of the memory (1024 points of 64 x 32
+// slabs take a twenty-fifth).
 //
 // Kept products take about half as much again.  They stay where 32 points with them
 // fit the device, a rule on device and shape only, so that a point's results
@@ -34,12 +36,13 @@ struct BatchPlan {
 template <class Bytes>
 BatchPlan plan_batch(int npts, int nmax, size_t avail, size_t total, size_t extra, int fixed, Bytes bytes) {
     const size_t budget = (size_t)(0.80 * (double)avail), kept = extra > 0 ? std::min(extra, budget) : budget;
+    const size_t wide = std::min(kept, total / 16);
     const int tiles = ((nmax + 63) / 64) * ((nmax + 63) / 64);
     const int base = std::min(npts, 128), most = std::min(npts, std::max(128, 1024 / tiles));
     auto points = [&](bool keep) {
         if (fixed > 0) return std::min(npts, fixed);
         int B = most;
-        while (B > base && bytes(B, keep) > kept) B = B * 3 / 4;
+        while (B > base && bytes(B, keep) > wide) B = B * 3 / 4;
         B = std::max(B, base);
         while (B > 1 && bytes(B, keep) > budget) B = B * 3 / 4;
         return std::max(B, 1);

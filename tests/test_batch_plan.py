@@ -1,5 +1,6 @@
 """The points per device batch and the choice to keep the first pass's products (csrc/qt_plan.h, compiled for
-the host): a call that fits the memory without the kept products fits with the plan."""
+the host): a call that fits the memory without the kept products fits with the plan, and blocks that take
+more than 128 points leave the rest of the device alone."""
 import itertools
 import os
 import subprocess
@@ -50,6 +51,7 @@ def _workspace(per, B, keep):
     ((1000, 64, TOTAL, TOTAL, 0, 0, 8 << 20), (1000, True)),     # small blocks: up to 1024 points
     ((200, 64, TOTAL, TOTAL, 0, 0, 8 << 20), (200, True)),
     ((300, 96, TOTAL, TOTAL, 0, 0, 8 << 20), (150, True)),       # 256 points at most, dealt evenly
+    ((1000, 64, TOTAL, TOTAL, 0, 0, 256 << 20), (125, True)),    # ... but a sixteenth of the memory at most
     ((64, 512, 36 * GB, TOTAL, 0, 0, GB), (22, False)),          # short of memory: 22 points a batch, 16 with X and V
     ((64, 512, GB, TOTAL, 0, 0, 9 * GB // 10), (1, False)),      # one point fits without them only
     ((64, 512, 36 * GB, TOTAL, 0, 28, GB), (28, False)),         # fixed points fit without them only
@@ -75,6 +77,7 @@ def test_plan_fits_where_the_plain_sweep_does(plan):
             assert B == min(npts, fixed), row
         else:
             assert _workspace(per, B, keep) <= budget or (B, keep) == (1, False), row
+            assert B <= 128 or _workspace(per, B, keep) <= total // 16, row
             assert -(-npts // B) * B - npts < -(-npts // B), row  # padding: less than a point a batch
         if keep:
             assert _workspace(per, B, True) <= min(extra or budget, budget), row
