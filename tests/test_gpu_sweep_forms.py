@@ -3,7 +3,8 @@ devices whose neighbouring slabs take the Z form (equal sizes) and the other
 one in turn, couplings that differ from slab to slab (the first pass's products
 are then not those of the reference's forward second pass), and diagonals that
 do not depend on whether the blocks are asked for too, and the sweep without the
-first pass's products (memory refused).  The contacts are
+first pass's products (memory refused), and scattering self-energies whose Sigma^<
+is not anti-Hermitian.  The contacts are
 broadened by 10 meV; every point is held to the parity bar of the sweep tests,
 relative to the largest block of the recursion."""
 import numpy as np
@@ -26,18 +27,21 @@ def qt():
     return rgf
 
 
-def _recursion(oracle_mod, Hii, H1i, E, fwd, fix, mul=0.0, mur=-0.1, T=300.0):
+def _recursion(oracle_mod, Hii, H1i, E, fwd, fix, mul=0.0, mur=-0.1, T=300.0, sr=None, sl=None):
     """rgf_mod.f90:46-472 for one point: diagonals of G^R, G^< and the
-    currents at the last and the first contact of the first pass."""
+    currents at the last and the first contact of the first pass.  sr, sl:
+    scattering self-energies per slab (:120-133)."""
+    inj0 = [0.0] * len(Hii) if sl is None else sl
+    Hii = Hii if sr is None else [np.asfortranarray(h + x) for h, x in zip(Hii, sr)]
     nx = len(Hii)
     ferm = lambda mu: 1.0 / (1.0 + np.exp((E - mu) / (8.61734e-05 * T)))
     fF, fL = ferm(mur), ferm(mul)
     order = list(range(nx)) if fwd else list(range(nx - 1, -1, -1))
-    sf, sl = order[0], order[-1]
+    sf, last_s = order[0], order[-1]
     uF, uL = (H1i[0], H1i[nx]) if fwd else (H1i[nx], H1i[0])
     lead = lambda h, u: oracle_mod.sancho(None, h, np.asfortranarray(u), E, eta=ETA, nmax=50)[0]
     sigF = uF @ lead(Hii[sf], H_(uF) if fwd else uF) @ H_(uF)
-    sigL = H_(uL) @ lead(Hii[sl], uL if fwd else H_(uL)) @ uL
+    sigL = H_(uL) @ lead(Hii[last_s], uL if fwd else H_(uL)) @ uL
     gl, gln, prev = {}, {}, None
     for s in order:
         if prev is None:
@@ -45,34 +49,36 @@ def _recursion(oracle_mod, Hii, H1i, E, fwd, fix, mul=0.0, mur=-0.1, T=300.0):
         else:
             u = H1i[s if fwd else s + 1]
             sig, inj = u @ gl[prev] @ H_(u), u @ gln[prev] @ H_(u)
-        if s == sl:
+        inj = inj + inj0[s]
+        if s == last_s:
             sig, inj = sig + sigL, inj - (sigL - H_(sigL)) * fL
         gl[s] = np.linalg.inv(E * np.eye(len(Hii[s])) - Hii[s] - sig)
         gln[s] = gl[s] @ inj @ H_(gl[s])
         prev = s
-    G, L = {sl: gl[sl]}, {sl: gln[sl]}
+    G, L = {last_s: gl[last_s]}, {last_s: gln[last_s]}
     for q, s in zip(order[:0:-1], order[-2::-1]):
         w = H1i[s + 1 if fwd and fix else s]
         x = gl[s] @ H_(w)
         G[s] = gl[s] + x @ G[q] @ w @ gl[s]
-        t = x @ G[q] @ w @ gln[s]
-        L[s] = gln[s] + x @ L[q] @ H_(x) + t - H_(t)
+        xg = x @ G[q]
+        L[s] = gln[s] + x @ L[q] @ H_(x) + xg @ w @ gln[s] + gln[s] @ H_(w) @ H_(xg)
     cur = lambda sig, s, f: np.trace(-(sig - H_(sig)) @ (L[s] + f * (G[s] - H_(G[s])))).real
     diag = lambda A: np.concatenate([np.diagonal(A[s]) for s in range(nx)])
-    last, first = cur(sigL, sl, fL), cur(sigF, sf, fF)
+    last, first = cur(sigL, last_s, fL), cur(sigF, sf, fF)
     # what rounding errors scale with: the connected blocks are nearly singular
     # where their partial chain has a level, and enter G by cancellation
     big = max(np.abs(a[s]).max() for a in (gl, gln, G) for s in range(nx))
     return diag(G), diag(L), (last if fwd else first), (first if fwd else last), big
 
 
-def _check(qt, oracle_mod, dev, variant="forward", fix=False):
+def _check(qt, oracle_mod, dev, variant="forward", fix=False, sr=None, sl=None):
     E = hm.energy_grid(-0.25, 0.15, 5)  # around the two chemical potentials
     H = qt.Hamiltonian.from_device(dev)
-    r = qt.solve_batch(H, E, None, variant=variant, mul=0.0, mur=-0.1, coupling_fix=fix, lead_eta=ETA)
+    r = qt.solve_batch(H, E, None, variant=variant, mul=0.0, mur=-0.1, coupling_fix=fix, lead_eta=ETA,
+                       sigma_lesser_ph=sl and [sl] * len(E), sigma_r_ph=sr and [sr] * len(E))
     H.close()
     for i, e in enumerate(E):
-        g, l, tr, tre, big = _recursion(oracle_mod, dev.Hii[0], dev.H1i[0], e, variant == "forward", fix)
+        g, l, tr, tre, big = _recursion(oracle_mod, dev.Hii[0], dev.H1i[0], e, variant == "forward", fix, sr=sr, sl=sl)
         for got, want in ((r["gr_diag"][i], g), (r["gl_diag"][i], l), (r["gg_diag"][i], l + g - g.conj())):
             assert np.abs(got - want).max() <= BAR * big
         scale = big * len(dev.Hii[0][0])
@@ -123,3 +129,18 @@ def test_products_not_kept(qt, oracle_mod, monkeypatch, sizes, variant):
     qt.solve_batch(H, hm.energy_grid(-0.25, 0.15, 140), None, variant=variant, coupling_fix=uneven, lead_eta=ETA)
     H.close()
     assert qt.last_timing()["batch"] == 70
+
+
+@pytest.mark.parametrize("workset", [None, "1"])
+@pytest.mark.parametrize("sizes,variant", [([33] * 5, "forward"), ([65] * 4, "backward"), ([20, 20, 64, 64, 33], "forward")])
+def test_scattering(qt, oracle_mod, monkeypatch, sizes, variant, workset):
+    if workset:
+        monkeypatch.setenv("QT_WORKSET_BYTES", workset)
+    uneven = len(set(sizes)) > 1
+    dev = (hm.uneven_device(sizes, seed=23, coupling_density=0.2) if uneven
+           else hm.synthetic_device(sizes[0], len(sizes), seed=31, coupling_density=0.2)[1])
+    rng = np.random.default_rng(41)
+    cr = lambda n: rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))
+    sr = [0.02 * cr(n) / np.sqrt(n) - 0.05j * np.eye(n) for n in sizes]
+    sl = [0.03 * cr(n) / np.sqrt(n) + 0.02j * np.eye(n) for n in sizes]
+    _check(qt, oracle_mod, dev, variant, fix=uneven, sr=sr, sl=sl)
