@@ -554,7 +554,7 @@ template <int NW>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void gj_step_kernel(
     double2* A, int64_t sa, const double2* Gprev, double2* Gm, int64_t sg, int n, int batch, int npan, int ntiles,
     int kprev, int kb, int* pivp, int* info, const int* active) {
-    constexpr int NB = kLaNB, R = 1, NT = NW * 64, NTL = NB / 16, NG = NB / 4, RB = 4 * R, NR = NW * R * 64;
+    constexpr int NB = kLaNB, NT = NW * 64, NTL = NB / 16, NG = NB / 4, RB = 4;
     static_assert(NW <= 8, "at most 32 row groups");
     // LDS: the replay's arrays are dead once the panel is factored
     struct Replay {
@@ -567,7 +567,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
         double2 raw[2][4][NB];      // the group's pivot rows before the group
         double2 yb[2][4][NB];       // their values when they were eliminated with
         double2 dfac[NB];           // 1 / pivot of step c
-        double2 gx[4][NR];          // the group's columns / multipliers between the two layouts
+        double2 gx[4][NT];          // the group's columns / multipliers between the two layouts
         double cand[2][32];         // candidate key of each 16-lane row, by step parity
         int pcol[NB];               // pivot row of step c
     };
@@ -578,7 +578,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     __shared__ unsigned used[32];   // rows pivoted before this panel (n <= 1024)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int li = lane & 15, lk = lane >> 4;
-    const int row0 = wave * R * 64;  // the wave's first row
+    const int row0 = wave * 64;  // the wave's first row
     const int wprev = kprev >= 0 ? min(NB, n - kprev) : 0;
 
     if ((int)blockIdx.x >= npan) {  // ---- replay on one tile
@@ -662,14 +662,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     auto& gx = sm.p.gx;
     for (int e = tid; e < 64; e += NT) cand[e >> 5][e & 31] = 0.0;
     __syncthreads();
-    bool mine[R];   // row row0 + 64 r + lane not yet pivoted
-    int ppos[R];    // step of this panel that pivoted it, -1 if none
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int row = row0 + r * 64 + lane;
-        mine[r] = row < n && !((used[(row >> 5) & 31] >> (row & 31)) & 1u);
-        ppos[r] = -1;
-    }
+    const int row = row0 + lane;  // this lane's row where a row is a lane's
+    bool mine = row < n && !((used[(row >> 5) & 31] >> (row & 31)) & 1u);  // not yet pivoted
+    int ppos = -1;                // step of this panel that pivoted it, -1 if none
     int zero_col = 0;  // first zero pivot (1-based), uniform
 
 #pragma unroll 1
@@ -686,16 +681,12 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
                 for (int i = 0; i < RB; ++i)
                     gx[lk][row0 + i * 16 + li] = make_double2(accR[i][s / 4][s % 4], accI[i][s / 4][s % 4]);
             }
-        double2 cur[R][4], am[R][4], dloc[4];
+        double2 cur[4], am[4], dloc[4];
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                cur[r][c] = gx[c][row0 + r * 64 + lane];
-                am[r][c] = make_double2(0.0, 0.0);
-            }
-#pragma unroll
-        for (int c = 0; c < 4; ++c) dloc[c] = make_double2(0.0, 0.0);
+        for (int c = 0; c < 4; ++c) {
+            cur[c] = gx[c][row];
+            am[c] = dloc[c] = make_double2(0.0, 0.0);
+        }
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             if (c >= nc) break;  // uniform
@@ -705,28 +696,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
             // bits (positive doubles order as their bits).  An infinite entry
             // counts as the largest finite one; 0 for rows already pivoted and
             // for a NaN, so that every key is a number
-            double key = 0.0;
-            double2 best[4];
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int row = row0 + r * 64 + lane;
-                const double a = cabs1(cur[r][c]);
-                const int hi = __double2hiint(a), lo = hi > 0x7fefffff ? ~0 : __double2loint(a);
-                double k = __hiloint2double(min(hi, 0x7fefffff), (lo & ~1023) | (1023 - row));
-                k = mine[r] && a == a ? k : 0.0;
-                const bool up = r == 0 || k > key;
-                key = up ? k : key;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    best[e].x = up ? cur[r][e].x : best[e].x;
-                    best[e].y = up ? cur[r][e].y : best[e].y;
-                }
-            }
+            const double a = cabs1(cur[c]);
+            const int hi = __double2hiint(a), lo = hi > 0x7fefffff ? ~0 : __double2loint(a);
+            double key = __hiloint2double(min(hi, 0x7fefffff), (lo & ~1023) | (1023 - row));
+            key = mine && a == a ? key : 0.0;
             const double kmax = row16_max(key);
             if (key == kmax) {
                 cand[buf][wave * 4 + lk] = key;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) crow[buf][wave * 4 + lk][e] = best[e];
+                for (int e = 0; e < 4; ++e) crow[buf][wave * 4 + lk][e] = cur[e];
             }
             __syncthreads();
             const double top = row16_max(NW > 4 ? fmax(cand[buf][li], cand[buf][16 + li]) : cand[buf][li]);
@@ -734,7 +712,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
             int p = 1023 - (tlo & 1023);
             const bool none = p >= n;  // top = 0: every row left is a NaN
             p = none ? 0 : p;
-            const int pw = p / (64 * R);  // its wave
+            const int pw = p / 64;  // its wave
             const int slot = pw * 4 + ((p >> 4) & 3);
             double2 u[4];
 #pragma unroll
@@ -745,83 +723,64 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
                 zero_col = zero_col == 0 ? kb + 4 * g + c + 1 : zero_col;
             }
             dloc[c] = d;
+            const double2 gf = cmul(cur[c], d);  // f / pivot
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const double2 gf = cmul(cur[r][c], d);  // f / pivot
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if (e == c) continue;
-                    double2 t = cur[r][e];
-                    t.x = fma(-gf.x, u[e].x, t.x);
-                    t.x = fma(gf.y, u[e].y, t.x);
-                    t.y = fma(-gf.x, u[e].y, t.y);
-                    t.y = fma(-gf.y, u[e].x, t.y);
-                    cur[r][e] = t;
-                }
-                cur[r][c] = make_double2(-gf.x, -gf.y);
-                am[r][c] = gf;
+            for (int e = 0; e < 4; ++e) {
+                if (e == c) continue;
+                double2 t = cur[e];
+                t.x = fma(-gf.x, u[e].x, t.x);
+                t.x = fma(gf.y, u[e].y, t.x);
+                t.y = fma(-gf.x, u[e].y, t.y);
+                t.y = fma(-gf.y, u[e].x, t.y);
+                cur[e] = t;
             }
-            if (pw == wave) {  // the pivot row itself stays, unscaled
+            cur[c] = make_double2(-gf.x, -gf.y);
+            am[c] = gf;
+            if (pw == wave && row == p) {  // the pivot row itself stays, unscaled
 #pragma unroll
-                for (int r = 0; r < R; ++r)
-                    if (row0 + r * 64 + lane == p) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) cur[r][e] = e == c ? make_double2(1.0, 0.0) : u[e];
-                        am[r][c] = make_double2(0.0, 0.0);
-                        mine[r] = false;
-                        ppos[r] = 4 * g + c;
-                        pcol[4 * g + c] = p;
-                        dfac[4 * g + c] = d;
-                    }
+                for (int e = 0; e < 4; ++e) cur[e] = e == c ? make_double2(1.0, 0.0) : u[e];
+                am[c] = make_double2(0.0, 0.0);
+                mine = false;
+                ppos = 4 * g + c;
+                pcol[4 * g + c] = p;
+                dfac[4 * g + c] = d;
             }
         }
         // multipliers for the update of the other columns (the pivot row of
         // step c carries 1 / pivot_c there), and of the pivot rows for y
+        if (row < n) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int row = row0 + r * 64 + lane;
-            if (row < n) {
+            for (int c = 0; c < 4; ++c) {
+                const bool own = ppos == 4 * g + c;
+                double2 rec;
+                rec.x = own ? dloc[c].x : am[c].x;
+                rec.y = own ? dloc[c].y : am[c].y;
+                if (c < nc) Gb[(unsigned)((4 * g + c) * n + row)] = rec;
+            }
+            if (ppos >= 4 * g) {
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const bool own = ppos[r] == 4 * g + c;
-                    double2 rec;
-                    rec.x = own ? dloc[c].x : am[r][c].x;
-                    rec.y = own ? dloc[c].y : am[r][c].y;
-                    if (c < nc) Gb[(unsigned)((4 * g + c) * n + row)] = rec;
-                }
-                if (ppos[r] >= 4 * g) {
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) lrow[par][ppos[r] - 4 * g][c] = am[r][c];
-                }
+                for (int c = 0; c < 4; ++c) lrow[par][ppos - 4 * g][c] = am[c];
             }
         }
         // back to the matrix layout: first the multipliers, then the columns
         double2 gm[RB], gc[RB];
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {  // (a pivot row takes the later steps only)
-                const bool before = c < ppos[r] - 4 * g;
-                gx[c][row0 + r * 64 + lane] =
-                    make_double2(before ? 0.0 : am[r][c].x, before ? 0.0 : am[r][c].y);
-            }
+        for (int c = 0; c < 4; ++c) {  // (a pivot row takes the later steps only)
+            const bool before = c < ppos - 4 * g;
+            gx[c][row] = make_double2(before ? 0.0 : am[c].x, before ? 0.0 : am[c].y);
+        }
 #pragma unroll
         for (int i = 0; i < RB; ++i) gm[i] = gx[lk][row0 + i * 16 + li];
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) gx[c][row0 + r * 64 + lane] = cur[r][c];
+        for (int c = 0; c < 4; ++c) gx[c][row] = cur[c];
 #pragma unroll
         for (int i = 0; i < RB; ++i) gc[i] = gx[lk][row0 + i * 16 + li];
         // the pivot rows as they were before the group, by the wave that holds them
-        bool any = false;
-#pragma unroll
-        for (int r = 0; r < R; ++r) any = any || ppos[r] >= 4 * g;
-        const bool hold = __ballot(any) != 0;
+        const bool hold = __ballot(ppos >= 4 * g) != 0;
         if (hold) {
 #pragma unroll
             for (int i = 0; i < RB; ++i) {
-                const int pp = __shfl(ppos[i / 4], (i % 4) * 16 + li, 64) - 4 * g;
+                const int pp = __shfl(ppos, i * 16 + li, 64) - 4 * g;
                 if (pp >= 0) {
 #pragma unroll
                     for (int t = 0; t < NTL; ++t)
@@ -859,7 +818,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
                 yb[par][lk][16 * t + li] = make_double2(-bn.x, -bn.y);
 #pragma unroll
                 for (int i = 0; i < RB; ++i) {
-                    const int pp = __shfl(ppos[i / 4], (i % 4) * 16 + li, 64) - 4 * g;
+                    const int pp = __shfl(ppos, i * 16 + li, 64) - 4 * g;
                     if (pp >= 0) {
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
@@ -896,7 +855,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
     if (tid < ncols) pv[kb + tid] = pcol[tid];
 #pragma unroll
     for (int i = 0; i < RB; ++i) {
-        const int pp = __shfl(ppos[i / 4], (i % 4) * 16 + li, 64);
+        const int pp = __shfl(ppos, i * 16 + li, 64);
         const int row = row0 + i * 16 + li;
         if (row >= n) continue;
         const double2 d = pp >= 0 ? dfac[pp] : make_double2(1.0, 0.0);
