@@ -182,7 +182,7 @@ struct Work {
 size_t work_bytes(const qt_ham& h, int B, bool sigma, bool keep = false);
 void work_carve(Arena& a, Work& w, const qt_ham& h, int B, bool sigma, bool keep = false);
 void inv_batch(Ctx& c, Work& w, int n, int batch, double2* A, int64_t sa, double2* X, int64_t sx,
-               const int* active, int flop_batch = -1, bool lookahead = true);
+               const int* active, int flop_batch = -1, bool free_rounding = true);
 void note_inv_info(Ctx& c, Work& w, int batch, int period);
 
 // ------------------------------------------------------------ Sancho-Rubio

@@ -619,8 +619,7 @@ void launch_wide(hipStream_t s, const ZGemmArgs& a) {
 }
 
 // Tile choice.  QT_GEMM_TILE=64x64, 128x64, 128x64w8, 32x32 or 32x32k8 fixes the
-// kernel;
-// otherwise the autotuner below picks per shape (QT_GEMM_TUNE=0: the
+// kernel; otherwise the autotuner below picks per shape (QT_GEMM_TUNE=0: the
 // row-waste rule of use_wide alone).  All kernels accumulate every
 // output element in the same order (k ascending in groups of 4, the same
 // MFMAs per group and component, the same epilogue), so the choice never
@@ -665,7 +664,8 @@ bool use_wide(int M) {
 // only read; at most 512 MiB of scratch, fewer members where the full batch
 // needs more) after the work already queued on the stream, and the faster
 // kernel is kept for the shape for the life of the process.  Where the
-// scratch cannot be allocated the row-waste rule decides.
+// scratch cannot be allocated the row-waste rule decides; it knows 64- and
+// 128-row tiles only, so that 32x32 ones run where they were timed.
 struct TuneState {
     std::mutex mu;
     std::map<std::tuple<int, int, int, int, int>, int> tile;

@@ -82,9 +82,9 @@ struct InvArgs {
     int64_t sg = 0;             // >= n * kInvPanelMax
     const int* active = nullptr;
     int flop_batch = -1;        // members counted by the timer (-1: batch)
-    // blocks of 65..384 by the look-ahead steps (X is their scratch: not A, sx >= 64 n), those up to 64 with
-    // the shorter reciprocal
-    bool lookahead = false;
+    // the result need not carry the panel kernels' rounding: blocks of 65..384 by the look-ahead steps (X is
+    // their scratch: not A, sx >= 64 n), those up to 64 with the shorter reciprocal
+    bool free_rounding = false;
 };
 void zinv(hipStream_t s, const InvArgs& a, Timer* t);
 // The same inversion with every member on stream s: no side streams, no

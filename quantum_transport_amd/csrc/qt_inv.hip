@@ -28,14 +28,17 @@
 //      other rows were eliminated with, which is what gives Gauss-Jordan its
 //      small residual |A X - I|; multiplying by the panel's explicit
 //      inv(A_KK) instead loses up to cond(A_KK) of it.
-// Blocks of 65 to 384 take, where the caller allows it (InvArgs::lookahead), one
+// Blocks of 65 to 384 take, where the caller allows it (InvArgs::free_rounding), one
 // launch per panel instead (gj_step_kernel): the panel's workgroups bring their
 // columns up to date and factor them while others replay the panel before.
+// Its pivot is the first row among those whose |re| + |im| equals the maximum in
+// all but the last ten bits (2.3e-13 of it at most): rows that close to a tie can
+// be taken in another order than by IZAMAX, with the same growth bound.
 // Blocks of n <= 64 are inverted by one kernel holding the whole matrix in
-// registers (gj_small_kernel: the same pivot rule and row operations, no
-// panel records).
-// A zero pivot sets info (first column, 1-based) and the output block is
-// zeroed (linalg.f90:50-58).
+// registers (gj_small_kernel: the panel kernel's pivot rule and row operations,
+// no panel records).
+// A column without a pivot (zero, or all its rows left are NaN) sets info (first
+// column, 1-based) and the output block is zeroed (linalg.f90:50-58).
 #include <algorithm>
 #include <cfloat>
 #include <climits>
@@ -545,11 +548,17 @@ __device__ __forceinline__ void replay_block(const double2* Gb, int n, int w, in
 // rows in LDS; a pivot row starts from its own y and takes the later steps, the
 // row operations of the unblocked elimination in their order.
 //
-// Bound by the panel's chain: some 1400 cycles a column (search, barrier,
-// reciprocal, update) and 5900 a group for turning and matrix work.  One
-// stream: 48 members of 250 0.888 -> 0.731 ms, 60 of 192 0.645 -> 0.559, 32 of
-// 384 1.55 -> 1.29, 48 of 300 1.24 -> 1.07; at 512 the two are level (the panel's
-// eight waves share the matrix cores of one CU), so the line lies at 384.
+// Bound by the panel's workgroup.  By cycle counter at n = 300 (48 members; 96
+// and 192 in brackets) a panel takes 194 k cycles: 74 k (53, 69) to load it and
+// replay the panel before on it, 50 k for its columns' chain of search, barrier,
+// reciprocal and update (1550 a column; 1270, 1450), 68 k for the rest of its
+// eight groups: 2.6 k a group to turn the columns, record and turn back, 4.5 k
+// (4.0, 3.6) for y and the matrix cores, 1.5 k at the loop's head.
+//
+// One stream, against panel and update in launches of their own: 48 members of
+// 250 0.888 -> 0.736 ms, 60 of 192 0.645 -> 0.558, 32 of 384 1.55 -> 1.27, 48 of
+// 300 1.24 -> 1.02; at 512 the two are level (the panel's eight waves share the
+// matrix cores of one CU), so the line lies at 384.
 template <int NW>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2))) void gj_step_kernel(
     double2* A, int64_t sa, const double2* Gprev, double2* Gm, int64_t sg, int n, int batch, int npan, int ntiles,
@@ -920,7 +929,7 @@ __global__ __launch_bounds__(256) void gj_finish_kernel(const double2* W, int64_
 //
 // Bound by the column's chain (search, barrier, reciprocal, readlanes).  Eight
 // columns a wave instead of sixteen leave 32 x 32 blocks half the readlanes: one
-// block, call included, 52 -> 43 us; FAST (InvArgs::lookahead) takes one
+// block, call included, 52 -> 43 us; FAST (InvArgs::free_rounding) takes one
 // refined reciprocal instead of Smith's three dependent divisions: 41 us, and
 // 256 of 64 x 64 88 -> 81 us.
 __device__ __forceinline__ double readlane_f64(double x, int l) {
@@ -1077,14 +1086,14 @@ void zinv_part(hipStream_t s, const InvArgs& a) {
             hipLaunchKernelGGL(kernel, dim3(a.batch), dim3(64 * waves), 0, s, a.A, a.sa, a.X, a.sx, n, a.info, a.active);
         };
         if (n <= 32)
-            a.lookahead ? launch(gj_small_kernel<4, true>, 4) : launch(gj_small_kernel<4, false>, 4);
+            a.free_rounding ? launch(gj_small_kernel<4, true>, 4) : launch(gj_small_kernel<4, false>, 4);
         else
-            a.lookahead ? launch(gj_small_kernel<8, true>, 8) : launch(gj_small_kernel<8, false>, 8);
+            a.free_rounding ? launch(gj_small_kernel<8, true>, 8) : launch(gj_small_kernel<8, false>, 8);
         QT_HIP(hipGetLastError());
         return;
     }
     hipLaunchKernelGGL(zero_int_kernel, dim3((a.batch + 255) / 256), dim3(256), 0, s, a.info, a.batch);
-    if (a.lookahead && n <= kLaMax) {
+    if (a.free_rounding && n <= kLaMax) {
         switch ((n + 63) / 64) {
             case 2: run_steps<2>(s, a); break;
             case 3: run_steps<3>(s, a); break;
@@ -1117,7 +1126,6 @@ InvArgs members(const InvArgs& a, int b0, int cnt) {
     return h;
 }
 
-// a second stream (default priority) and two events for splitting a batch
 // up to three more streams (default priority) and their events for splitting
 // a batch; QT_INV_PARTS (2..4, default 2) sets the number of parts
 constexpr int kMaxParts = 4;
@@ -1151,14 +1159,6 @@ int inv_parts() {
 
 }  // namespace
 
-// Blocks of n <= 64 take the one-launch kernel above on stream s, the look-ahead
-// steps overlap their own panels with the matrix work, and up to n = 256 the
-// panels of all members run at once (a split there costs: 100 members of 160
-// in the sweep's decimation, whole call 51.4 -> 47.5 ms without it).  For larger
-// blocks the panel kernel keeps one workgroup per member busy for a whole latency-
-// bound column sweep, leaving most CUs idle; the batch is therefore split in
-// parts on as many streams so that the panels of one part run while the
-// MFMA updates of the others fill the remaining CUs.
 void zinv_single(hipStream_t s, const InvArgs& a) {
     if (a.n <= 0 || a.batch <= 0) return;
     if (a.n > 1024) throw hip_error("zinv: block size above 1024", 6);
@@ -1166,13 +1166,23 @@ void zinv_single(hipStream_t s, const InvArgs& a) {
     zinv_part(s, a);
 }
 
+// Blocks of n <= 64 take the one-launch kernel above on stream s, the look-ahead
+// steps overlap their own panels with the matrix work, and up to n = 256 the
+// panels of all members run at once: split over two streams they cost 17-27% at
+// 8 to 32 members (8 of 96 0.260 -> 0.308, 32 of 160 0.444 -> 0.548, of 200 0.590 ->
+// 0.750, of 256 0.755 -> 0.923 ms) and 5-28% at 64 to 200 (100 of 160 0.567 ->
+// 0.692, 128 of 256 1.33 -> 1.41; 128 of 200 alone gain 2%).  For larger
+// blocks the panel kernel keeps one workgroup per member busy for a whole latency-
+// bound column sweep, leaving most CUs idle; the batch is therefore split in
+// parts on as many streams so that the panels of one part run while the
+// MFMA updates of the others fill the remaining CUs.
 void zinv(hipStream_t s, const InvArgs& a, Timer* t) {
     const int n = a.n;
     if (n <= 0 || a.batch <= 0) return;
     if (n > 1024) throw hip_error("zinv: block size above 1024", 6);
     if (!a.G || a.sg < (int64_t)n * kInvPanelMax) throw hip_error("zinv: multiplier workspace missing", 1);
     if (t && t->enabled) t->begin(s, 1);
-    if (a.batch >= 8 && n > 256 && !(a.lookahead && n <= kLaMax)) {
+    if (a.batch >= 8 && n > 256 && !(a.free_rounding && n <= kLaMax)) {
         Side& sd = side();
         const int parts = std::min(inv_parts(), a.batch / 4);
         QT_HIP(hipEventRecord(sd.fork, s));

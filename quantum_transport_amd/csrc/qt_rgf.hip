@@ -113,7 +113,7 @@ void work_carve(Arena& a, Work& w, const qt_ham& h, int B, bool sigma, bool keep
 }
 
 void inv_batch(Ctx& c, Work& w, int n, int batch, double2* A, int64_t sa, double2* X,
-               int64_t sx, const int* active, int flop_batch, bool lookahead) {
+               int64_t sx, const int* active, int flop_batch, bool free_rounding) {
     InvArgs a;
     a.n = n;
     a.batch = batch;
@@ -127,7 +127,7 @@ void inv_batch(Ctx& c, Work& w, int n, int batch, double2* A, int64_t sa, double
     a.sg = (int64_t)n * kInvPanelMax;
     a.active = active;
     a.flop_batch = flop_batch;
-    a.lookahead = lookahead;
+    a.free_rounding = free_rounding;
     zinv(c.stream, a, &c.timer);
 }
 
@@ -772,7 +772,7 @@ struct Solve {
         // With Z_i = X_i G_{i+1} W the full block is G_i = (I + Z_i) Gl_i, and G
         // itself is not needed to go on: G_i W = V_i + Z_i V_i with the V_i = Gl_i U
         // of the first pass.  So where only diagonals are asked for, a slab takes
-        // five products here (ten in all, with the inversion) instead of seven, G
+        // five products here (ten in both passes, beside the inversion) instead of seven, G
         // being formed at the contact, for callers that want its blocks, and
         // where the next slab needs it.  Measured, whole
         // sweeps (leads included): 512 x 20 slabs, 64 points 482.7 -> 446.3 ms; the GW
@@ -1038,8 +1038,7 @@ int qt_ham_create(int32_t nx, const int32_t* nm, int32_t nk, const void* const* 
         // neighbouring couplings that coincide (every Wannier-built device)
         h->csame.assign(nx + 1, 0);
         for (int s = 1; s < nx; ++s) {
-            const int prows = s - 1 < nx ? nm[s - 1] : nm[nx - 1], pcols = s == 1 ? nm[0] : nm[s - 2];
-            bool eq = nm[s] == prows && nm[s - 1] == pcols;
+            bool eq = nm[s] == nm[s - 1] && nm[s - 1] == (s == 1 ? nm[0] : nm[s - 2]);
             for (int k = 0; eq && k < nk; ++k) {
                 const void* a = H1i[(int64_t)k * (nx + 1) + s];
                 const void* b = H1i[(int64_t)k * (nx + 1) + s - 1];
@@ -1572,7 +1571,7 @@ int qt_invert_batched_noalloc(int32_t n, int32_t batch, void* A, void* X, int32_
         a.info = sinfo;  // cleared by the inversion itself
         a.G = G;
         a.sg = (int64_t)n * kInvPanelMax;
-        a.lookahead = true;
+        a.free_rounding = true;
         zinv_single(c.stream, a);
         hipLaunchKernelGGL(info_any_kernel, dim3((batch + 255) / 256), dim3(256), 0, c.stream, sinfo, batch,
                            flag);
