@@ -285,7 +285,7 @@ def run_ephoton(args) -> dict:
                        "nm": nm, "slabs": length, "energies": nen, "nop": nop},
             "roofline": {"bound": "mfma", "achieved": round(tf, 3), "peak": 78.6, "unit": "TFLOP/s",
                          "frac": round(tf / 78.6, 4), "traffic": None,
-                         "kernel": "whole call: eph_sum + 4 x zgemm_mfma_kernel + eph_retarded"},
+                         "kernel": "whole call: eph_sum + 4 x zgemm_mfma_*_kernel + eph_retarded"},
             "cpu_baseline": None if args.no_cpu else ephoton_cpu_baseline(args, nm, nop)}
 
 

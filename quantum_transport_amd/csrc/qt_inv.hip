@@ -550,10 +550,11 @@ __device__ __forceinline__ void replay_block(const double2* Gb, int n, int w, in
 //
 // Bound by the panel's workgroup.  By cycle counter at n = 300 (48 members; 96
 // and 192 in brackets) a panel takes 194 k cycles: 74 k (53, 69) to load it and
-// replay the panel before on it, 50 k for its columns' chain of search, barrier,
-// reciprocal and update (1550 a column; 1270, 1450), 68 k for the rest of its
-// eight groups: 2.6 k a group to turn the columns, record and turn back, 4.5 k
-// (4.0, 3.6) for y and the matrix cores, 1.5 k at the loop's head.
+// replay the panel before on it, 46 k for its columns' chain of search, barrier,
+// reciprocal and update (1550 a column; 1270, 1450), 64 k for the rest of its
+// groups of four (2.6 k each to turn the columns, record and turn back, 4.5 k
+// (4.0, 3.6) for y and the matrix cores, 1.5 k at the loop's head), 9 k to write
+// it back.
 //
 // One stream, against panel and update in launches of their own: 48 members of
 // 250 0.888 -> 0.736 ms, 60 of 192 0.645 -> 0.558, 32 of 384 1.55 -> 1.27, 48 of
